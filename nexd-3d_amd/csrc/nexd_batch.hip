@@ -149,15 +149,17 @@ struct Batch : BatchBase {
         int rc = 0;
         for (int i = 0; i < 3 && !rc; ++i) rc = dalloc(&q[i], S * 9 * ng);
         for (int i = 0; i < 3 && !rc && c.compensated; ++i) rc = dalloc(&qlo[i], S * 9 * ng);
-        if (!rc && c.attenuation) (rc = dalloc(&th[0], S * 18 * ng)) || (rc = dalloc(&th[1], S * 18 * ng));
+        // the recomputing RK2 kernels keep 6 rates in th[1] and no second paux
+        if (!rc && c.attenuation)
+            (rc = dalloc(&th[0], S * 18 * ng)) || (rc = dalloc(&th[1], S * (recompute() ? 6 : 18) * ng));
         if (!rc && c.timeint == NEXD_LSRK4) {
             rc = dalloc(&qres, S * 9 * ng);
             if (!rc && c.attenuation) rc = dalloc(&thres, S * 18 * ng);
             if (!rc && c.pml) rc = dalloc(&pres, S * 27 * ng);
         }
         if (!rc && c.pml)
-            (rc = dalloc(&paux[0], S * 27 * ng)) || (rc = dalloc(&paux[1], S * 27 * ng)) ||
-                (rc = dalloc(&pmlc, (size_t)nmat_sets() * 9 * ng)) || (rc = dalloc(&last_flux, S * 27 * np));
+            (rc = dalloc(&paux[0], S * 27 * ng)) || (recompute() ? 0 : (rc = dalloc(&paux[1], S * 27 * ng))) ||
+                (rc = dalloc(&pmlc, (size_t)nmat_sets() * 9 * ng)) || (rc = dalloc(&last_flux, S * 54 * np));
         if (!rc && c.pml)
             (rc = dalloc(&pml_on, S)) || (rc = dalloc(&blk_energy, S * ((size_t)c.nelem + 64))) ||
                 (rc = dalloc(&energy, S * c.nt));
@@ -216,6 +218,13 @@ struct Batch : BatchBase {
     // (src/timeloopMod.f90:482-516)
     bool energy_on() const { return cfg.energy && cfg.pml; }
 
+    // TVD RK2 with attenuation or (compat) PML: the kernels that recompute
+    // the element-local stage-1 values
+    bool recompute() const {
+        return nexd::recompute_rk2(cfg.timeint, cfg.attenuation != 0, cfg.pml != 0,
+                                   (cfg.compat & NEXD_COMPAT_PML_LAST_ELEMENT) != 0);
+    }
+
     int check_shot(int shot) {
         if (cfg.shared_material ? shot != 0 : (shot < 0 || shot >= cfg.nshot))
             return fail(NEXD_E_ARG, "shot out of range (shared materials use shot 0)");
@@ -240,6 +249,7 @@ struct Batch : BatchBase {
         a.w23 = f32w ? (R)(2.0f / 3.0f) : (R)(2.0 / 3.0);
         a.pml_compat = (cfg.compat & NEXD_COMPAT_PML_LAST_ELEMENT) ? 1 : 0;
         a.last_flux = last_flux;
+        a.last_flux1 = last_flux ? last_flux + (size_t)cfg.nshot * 27 * np : nullptr;
         a.D = D; a.DK = DK; a.LT = LT; a.fmask = fmask;
         a.metric = metric; a.fscale = fscale; a.frame = frame; a.matc = matc;
         a.nbr = nbr; a.ftype = ftype; a.anel = anel;
@@ -343,6 +353,26 @@ struct Batch : BatchBase {
     }
 
     template <int ORDER>
+    void last_flux_rk2_impl() {
+        const int last = cfg.nelem - 1;
+        hipLaunchKernelGGL((nexd::last_flux_rk2_kernel<ORDER, R>), dim3(cfg.nshot), dim3(64), 0, stream, q[0], q[1],
+                           paux[0], pmlc, matc, last, pmlcheck[last] ? 1 : 0, (int)ng,
+                           cfg.shared_material ? 0 : cfg.nelem * 8, cfg.shared_material ? 0 : 9, (R)cfg.dt,
+                           (const R *)dt_elem, last_flux + (size_t)cfg.nshot * 27 * np, last_flux);
+    }
+
+    // the last element's fluxes of both stages, between the stages
+    void last_flux_rk2_dispatch() {
+        switch (cfg.order) {
+            case 1: last_flux_rk2_impl<1>(); break;
+            case 2: last_flux_rk2_impl<2>(); break;
+            case 3: last_flux_rk2_impl<3>(); break;
+            case 4: last_flux_rk2_impl<4>(); break;
+            default: last_flux_rk2_impl<5>(); break;
+        }
+    }
+
+    template <int ORDER>
     void step_end_impl(int row_offset, int advance) {
         // one block per shot and 1024 of its receiver values
         const int chunks = cfg.nrec > 0 ? (cfg.nrec * 9 + 1023) / 1024 : 1;
@@ -367,6 +397,11 @@ struct Batch : BatchBase {
         R *qin, *qout, *thin, *thout, *pin, *pout;
         if (scheme == NEXD_EULER) {
             qin = q[0]; qout = q[1]; thin = th[0]; thout = th[0]; pin = paux[0]; pout = paux[0];
+        } else if (recompute()) {
+            // q ping-pongs; memory variables and PML auxiliaries stay in buffer 0
+            qin = q[irk - 1]; qout = q[2 - irk]; thin = thout = th[0]; pin = pout = paux[0];
+            a.rate_out = th[1]; a.rate_in = th[1];
+            a.recompute = irk;
         } else if (scheme == NEXD_RK2) {
             if (irk == 1) { qin = q[0]; qout = q[1]; thin = th[0]; thout = th[1]; pin = paux[0]; pout = paux[1]; }
             else { qin = q[1]; qout = q[0]; thin = th[1]; thout = th[0]; pin = paux[1]; pout = paux[0]; }
@@ -402,6 +437,8 @@ struct Batch : BatchBase {
         const bool pml = cfg.pml && n_pml > 0;
         for (int irk = 1; irk <= nrk; ++irk) {
             set_stage_buffers(a, irk);
+            // before the interior list's stage 2 overwrites the step-start field
+            if (pml && a.recompute == 2) last_flux_rk2_dispatch();
             // the interior list, then the PML list, on the one stream (a
             // captured fork onto a second stream keeps the buffers its
             // kernels use allocated after the graph and the buffers are
@@ -413,7 +450,7 @@ struct Batch : BatchBase {
             a.blk_energy = en ? blk_energy : nullptr;
             dispatch(a, false, stream);
             if (pml) {
-                if (a.pml_compat) last_flux_dispatch(a.qin, a.pin);
+                if (a.pml_compat && !a.recompute) last_flux_dispatch(a.qin, a.pin);
                 a.elist = elist_pml;
                 a.nlist = n_pml;
                 a.blk_energy = en ? blk_energy + nblocks(n_plain, false) : nullptr;
@@ -447,12 +484,12 @@ struct Batch : BatchBase {
         }
         if (cfg.attenuation)
             for (int i = 0; i < 2; ++i) {
-                int rc = put(th[i], std::vector<R>(S * 18 * ng, tiny));
+                int rc = put(th[i], std::vector<R>(S * (i && recompute() ? 6 : 18) * ng, tiny));
                 if (rc) return rc;
             }
         if (cfg.pml)
             for (int i = 0; i < 2; ++i) {
-                int rc = put(paux[i], std::vector<R>(S * 27 * ng, R(0)));
+                int rc = paux[i] ? put(paux[i], std::vector<R>(S * 27 * ng, R(0))) : 0;
                 if (rc) return rc;
             }
         if (qres) {
@@ -547,7 +584,8 @@ struct Batch : BatchBase {
         // every RK stage in turn, as the time loop runs them, after a stage-1
         // warm-up; the last element's fluxes are computed once beforehand
         set_stage_buffers(a, 1);
-        if (list == 1 && a.pml_compat) last_flux_dispatch(a.qin, a.pin);
+        if (list == 1 && a.recompute) last_flux_rk2_dispatch();
+        else if (list == 1 && a.pml_compat) last_flux_dispatch(a.qin, a.pin);
         dispatch(a, list == 1);
         if (hipEventRecord(ev0, stream) != hipSuccess) return fail(NEXD_E_HIP, "hipEventRecord failed");
         // the last stage writes its energy partials, as in the time loop

@@ -154,7 +154,8 @@ void dispatch_stage(int order, const StageArgs<double> &a, bool att, bool pml, h
 }
 
 // Where a step's kernels keep their scratch: the energy block partials
-// (nblk_total values) and the last element's 27 fluxes (27*Np values).
+// (nblk_total values) and the last element's 27 fluxes (27*Np values, with
+// the recomputing RK2 kernels followed by those of stage 1).
 // nexd_run uses the context's buffers, nexd_run_noalloc a static array.
 struct StepScratch {
     double *blk_energy;
@@ -175,6 +176,32 @@ void dispatch_last_flux(nexd_ctx *c, const double *qin, const double *pin, doubl
         case 3: launch_last_flux<3>(c, qin, pin, out); break;
         case 4: launch_last_flux<4>(c, qin, pin, out); break;
         default: launch_last_flux<5>(c, qin, pin, out); break;
+    }
+}
+
+// TVD RK2 with attenuation or (compat) PML: the kernels that recompute the
+// element-local stage-1 values
+bool recompute(const nexd_ctx *c) {
+    return nexd::recompute_rk2(c->cfg.timeint, c->cfg.attenuation != 0, c->cfg.pml != 0,
+                               (c->cfg.compat & NEXD_COMPAT_PML_LAST_ELEMENT) != 0);
+}
+
+template <int ORDER>
+void launch_last_flux_rk2(nexd_ctx *c, double *out) {
+    const int last = c->cfg.nelem - 1;
+    hipLaunchKernelGGL((nexd::last_flux_rk2_kernel<ORDER, double>), dim3(1), dim3(64), 0, c->stream, c->q[0], c->q[1],
+                       c->paux[0], c->pmlc, c->matc, last, c->pmlcheck[last] ? 1 : 0, (int)c->nglob, 0, 0, c->cfg.dt,
+                       (const double *)nullptr, out + 27 * c->np, out);
+}
+
+// the last element's fluxes of both stages, between the stages
+void dispatch_last_flux_rk2(nexd_ctx *c, double *out) {
+    switch (c->cfg.order) {
+        case 1: launch_last_flux_rk2<1>(c, out); break;
+        case 2: launch_last_flux_rk2<2>(c, out); break;
+        case 3: launch_last_flux_rk2<3>(c, out); break;
+        case 4: launch_last_flux_rk2<4>(c, out); break;
+        default: launch_last_flux_rk2<5>(c, out); break;
     }
 }
 
@@ -222,6 +249,7 @@ StageArgs<double> base_args(nexd_ctx *c) {
     a.w23 = f32w ? (double)(2.0f / 3.0f) : 2.0 / 3.0;
     a.pml_compat = (c->cfg.compat & NEXD_COMPAT_PML_LAST_ELEMENT) ? 1 : 0;
     a.last_flux = c->last_flux;
+    a.last_flux1 = c->last_flux ? c->last_flux + 27 * c->np : nullptr;
     a.D = c->D; a.DK = nullptr; a.LT = c->LT; a.fmask = c->fmask;   // FP64: no contravariant form
     a.metric = c->metric; a.fscale = c->fscale; a.frame = c->frame; a.matc = c->matc;
     a.nbr = c->nbr; a.ftype = c->ftype; a.anel = c->anel;
@@ -245,6 +273,11 @@ void stage_buffers(nexd_ctx *c, int irk, StageArgs<double> &a) {
     double *qin, *qout, *thin, *thout, *pin, *pout;
     if (scheme == NEXD_EULER) {
         qin = c->q[0]; qout = c->q[1]; thin = c->th[0]; thout = c->th[0]; pin = c->paux[0]; pout = c->paux[0];
+    } else if (recompute(c)) {
+        // q ping-pongs; memory variables and PML auxiliaries stay in buffer 0
+        qin = c->q[irk - 1]; qout = c->q[2 - irk]; thin = thout = c->th[0]; pin = pout = c->paux[0];
+        a.rate_out = c->th[1]; a.rate_in = c->th[1];
+        a.recompute = irk;
     } else if (scheme == NEXD_RK2) {
         if (irk == 1) { qin = c->q[0]; qout = c->q[1]; thin = c->th[0]; thout = c->th[1]; pin = c->paux[0]; pout = c->paux[1]; }
         else { qin = c->q[1]; qout = c->q[0]; thin = c->th[1]; thout = c->th[0]; pin = c->paux[1]; pout = c->paux[0]; }
@@ -281,9 +314,12 @@ void enqueue_step(nexd_ctx *c, const StepScratch &sc) {
     const bool pml = c->have_pml && c->pml_active && c->n_pml > 0;
     StageArgs<double> a = base_args(c);
     a.last_flux = sc.last_flux;
+    a.last_flux1 = sc.last_flux + 27 * c->np;
     const int nrk = c->nrk;
     for (int irk = 1; irk <= nrk; ++irk) {
         stage_buffers(c, irk, a);
+        // before the interior list's stage 2 overwrites the step-start field
+        if (pml && a.recompute == 2) dispatch_last_flux_rk2(c, sc.last_flux);
         const double *qin = a.qin, *pin = a.pin;
         // energy partials: the plain list's blocks first, then the PML list's
         // (every element is in the plain list once the PML is switched off)
@@ -296,7 +332,7 @@ void enqueue_step(nexd_ctx *c, const StepScratch &sc) {
         a.blk_energy = energy ? sc.blk_energy : nullptr;
         dispatch_stage(c->cfg.order, a, att, false, c->stream);
         if (pml) {
-            if (a.pml_compat) dispatch_last_flux(c, qin, pin, sc.last_flux);
+            if (a.pml_compat && !a.recompute) dispatch_last_flux(c, qin, pin, sc.last_flux);
             a.elist = c->elist_pml;
             a.nlist = c->n_pml;
             a.blk_energy = energy ? sc.blk_energy + nblocks(c->cfg.order, c->n_plain, att, false) : nullptr;
@@ -411,10 +447,13 @@ int nexd_create(const nexd_config *cfg, nexd_ctx **out) {
     const size_t ng = c->nglob;
     int rc = 0;
     for (int i = 0; i < 3 && !rc; ++i) rc = dalloc(c, &c->q[i], 9 * ng);
-    if (!rc && cfg->attenuation) (rc = dalloc(c, &c->th[0], 18 * ng)) || (rc = dalloc(c, &c->th[1], 18 * ng));
+    // the recomputing RK2 kernels keep 6 rates in th[1] and no second paux
+    const bool rcmp = recompute(c);
+    if (!rc && cfg->attenuation)
+        (rc = dalloc(c, &c->th[0], 18 * ng)) || (rc = dalloc(c, &c->th[1], (rcmp ? 6 : 18) * ng));
     if (!rc && cfg->pml)
-        (rc = dalloc(c, &c->paux[0], 27 * ng)) || (rc = dalloc(c, &c->paux[1], 27 * ng)) ||
-            (rc = dalloc(c, &c->pmlc, 9 * ng)) || (rc = dalloc(c, &c->last_flux, 27 * c->np));
+        (rc = dalloc(c, &c->paux[0], 27 * ng)) || (rcmp ? 0 : (rc = dalloc(c, &c->paux[1], 27 * ng))) ||
+            (rc = dalloc(c, &c->pmlc, 9 * ng)) || (rc = dalloc(c, &c->last_flux, 54 * c->np));
     if (!rc && cfg->track_displacement) rc = dalloc(c, &c->u_full, 3 * ng);
     if (!rc && cfg->timeint == NEXD_LSRK4) {
         rc = dalloc(c, &c->qres, 9 * ng);
@@ -604,11 +643,13 @@ int nexd_reset(nexd_ctx *c) {
     for (int i = 0; i < 3; ++i) HIPCHK(c, hipMemcpy(c->q[i], tiny.data(), sizeof(double) * 9 * ng, hipMemcpyHostToDevice));
     if (c->cfg.attenuation) {
         std::vector<double> t18(18 * ng, tiny_v);
-        for (int i = 0; i < 2; ++i) HIPCHK(c, hipMemcpy(c->th[i], t18.data(), sizeof(double) * 18 * ng, hipMemcpyHostToDevice));
+        for (int i = 0; i < 2; ++i)
+            HIPCHK(c, hipMemcpy(c->th[i], t18.data(), sizeof(double) * (i && recompute(c) ? 6 : 18) * ng, hipMemcpyHostToDevice));
     }
     if (c->cfg.pml) {
         std::vector<double> z(27 * ng, 0.0);
-        for (int i = 0; i < 2; ++i) HIPCHK(c, hipMemcpy(c->paux[i], z.data(), sizeof(double) * 27 * ng, hipMemcpyHostToDevice));
+        for (int i = 0; i < 2; ++i)
+            if (c->paux[i]) HIPCHK(c, hipMemcpy(c->paux[i], z.data(), sizeof(double) * 27 * ng, hipMemcpyHostToDevice));
     }
     if (c->u_full) HIPCHK(c, hipMemcpy(c->u_full, tiny.data(), sizeof(double) * 3 * ng, hipMemcpyHostToDevice));
     if (c->qres) {
@@ -677,7 +718,7 @@ int nexd_run_noalloc(nexd_ctx *c, int it_begin, int it_end, double *energy) {
     if (it_begin != c->step + 1) return fail(c, NEXD_E_ARG, "it_begin must be the next step");
     if (it_end < it_begin || it_end > c->cfg.nt) return fail(c, NEXD_E_ARG, "it_end out of range");
     // scratch: the energy block partials, then the last element's fluxes
-    const size_t need = (size_t)c->nblk_total + 27 * (size_t)c->np;
+    const size_t need = (size_t)c->nblk_total + 54 * (size_t)c->np;
     if (need > kScratchReals)
         return fail(c, NEXD_E_UNSUPPORTED, "nexd_run_noalloc: the mesh needs more scratch than the static 2^20 values "
                                            "(use nexd_run)");
@@ -812,7 +853,8 @@ int nexd_time_stage_kernel(nexd_ctx *c, int list, int nrep, double *avg_ms, int 
         dispatch_stage(c->cfg.order, a, att, list == 1, c->stream);
     };
     stage_buffers(c, 1, a);
-    if (list == 1 && a.pml_compat) dispatch_last_flux(c, a.qin, a.pin, c->last_flux);
+    if (list == 1 && a.recompute) dispatch_last_flux_rk2(c, c->last_flux);
+    else if (list == 1 && a.pml_compat) dispatch_last_flux(c, a.qin, a.pin, c->last_flux);
     one(1);
     HIPCHK(c, hipEventRecord(c->ev0, c->stream));
     for (int r = 0; r < nrep; ++r)

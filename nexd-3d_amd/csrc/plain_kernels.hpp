@@ -68,7 +68,11 @@ struct StageArgs {
     const R *pin;               // [27][nglob] PML f',g',h'
     const R *pbase;
     R *pout;
+    int recompute;              // 1: RK2 stage 1, 2: RK2 stage 2 of the recomputing kernels (host only)
+    R *rate_out;                // [6][nglob] memory-variable rates of stage 1 (recomputing kernels)
+    const R *rate_in;           // the same, read by stage 2
     const R *last_flux;         // [27][NP] fluxes of the last element (compat)
+    const R *last_flux1;        // the same of stage 1 (recomputing kernels, stage 2)
     int pml_compat;
     const R *D;                 // Dr/Ds/Dt as MFMA A-operand fragments [RT][KS][64]
     const R *DK;                // [Dr|Ds|Dt] as MFMA A-operand fragments [RTV][3KS][64] (PML)
@@ -248,6 +252,7 @@ constexpr double kLsrkB[5] = {1432997174477.0 / 9575080441755.0, 5161836677717.0
                               1720146321549.0 / 2090206949498.0, 3134564353537.0 / 4481467310338.0,
                               2277821191437.0 / 14882151754819.0};
 
+// RC is the stage the recomputing RK2 kernels are compiled for (0: any).
 template <typename R>
 struct RkStage {
     R wb, wx;    // wb * base + wx * (a + dt*rhs)
@@ -255,8 +260,10 @@ struct RkStage {
     bool ls;     // low-storage RK4
     R la, lb;    // its A and B of the stage
 };
-template <typename R>
+template <typename R, int RC = 0>
 __device__ __forceinline__ RkStage<R> rk_stage(int scheme, int irk, R w13, R w23, R lsa, R lsb) {
+    if constexpr (RC == 1) return {R(0), R(1), false, false, R(0), R(0)};
+    if constexpr (RC == 2) return {R(0.5), R(0.5), true, false, R(0), R(0)};
     if (scheme == 4) return {R(0), R(1), false, true, irk == 1 ? R(0) : lsa, lsb};
     if (irk == 1) return {R(0), R(1), false, false, R(0), R(0)};
     if (scheme == 2) return {R(0.5), R(0.5), true, false, R(0), R(0)};
@@ -277,10 +284,12 @@ __device__ __forceinline__ R rk_combine(const RkStage<R> &s, R a, R base, R rhs,
 // previous residual on entry and the new one on return; A_1 = 0, so the
 // stage-1 residual need only be finite), rk_combine otherwise (`res` is the
 // RK base and stays as it is).
-template <typename R, bool LS, bool WEIGHTED = false>
+template <typename R, bool LS, bool WEIGHTED = false, int RC = 0>
 __device__ __forceinline__ R rk_update(const RkStage<R> &s, R a, R &res, R rhs, R dt) {
 #pragma clang fp contract(off)
-    if constexpr (LS) {
+    if constexpr (RC == 1) {
+        return a + rhs * dt;
+    } else if constexpr (LS) {
         const R r = s.la * res + rhs * dt;
         res = r;
         return a + s.lb * r;
@@ -430,8 +439,9 @@ struct Shape {
         return ROWS_A * nt > nt * NV ? ROWS_A * nt : nt * NV;
     }
     // the face region also holds the last element's 27 fluxes in phase 1
+    // (of both stages in the recomputing stage 2)
     static constexpr int face_reals(int eb) {
-        return eb * NFC * SFN > (PML ? 27 * NP : 0) ? eb * NFC * SFN : 27 * NP;
+        return eb * NFC * SFN > (PML ? 54 * NP : 0) ? eb * NFC * SFN : 54 * NP;
     }
     static constexpr int off_metric(int eb) {
         const int f = off_face(eb) + face_reals(eb);
@@ -506,7 +516,30 @@ struct Mfma<double> {
 // LS: the low-storage RK4 instantiation (residuals read and written in
 // place of the RK base); the TVD schemes use LS = false.  VAR: the block
 // shape (Shape).
-template <int ORDER, bool ATT, bool PML, typename R, bool LS, int VAR = 0>
+//
+// RC: the recomputing kernels of TVD RK2 (1: its first stage, 2: its second;
+// 0: any stage of any scheme).  The kernel moves its bytes at the rate of a
+// large copy less the latency of its phases, and of the 63 values of a node
+// (FP32 compensated, PML and attenuation) only the 9 fields are read by other
+// elements between the stages.  The others' stage-1 values depend on their
+// own step-start values and little else, so stage 1 does not store them and
+// stage 2 forms them again instead of loading them:
+//   - f',g',h' advance by -alpha f' - d/k (f' + u), u the last element's
+//     flux, which is the same for every element (compat): stage 1 writes
+//     none of them (and needs no u), stage 2 loads the 27 step-start values,
+//     repeats the stage-1 update with the same operations, so to the same
+//     bits, and updates in place;
+//   - the 18 memory variables advance by w_i (g_c - theta_ic), where the 6
+//     rates g (lifted flux less strain rate) are common to the mechanisms:
+//     stage 1 writes g, stage 2 loads g and the step-start values.
+// Per node of the two stages 315 -> 237 values (FP32 compensated), 270 ->
+// 192 without the low parts.  Measured: a step of the 192,000-tet N = 4 box
+// (attenuation, PML, FP64) 6.41 -> 5.46 ms; of 8 FP32 compensated shots on
+// the 41,472-tet version 4.68 -> 4.11 ms, of 6 on 24,000 tets at N = 2 0.64
+// -> 0.58 ms.  Without compat u is the element's own flux of the stage-1
+// state, which stage 2 does not hold: RC = 0 stays for it, and for the
+// other schemes.
+template <int ORDER, bool ATT, bool PML, typename R, bool LS, int VAR = 0, int RC = 0>
 __global__ void __launch_bounds__((Shape<ORDER, ATT, PML, R, VAR>::NTHR), (Shape<ORDER, ATT, PML, R, VAR>::WPS))
 stage_kernel(StageArgs<R> a) {
     using S = Shape<ORDER, ATT, PML, R, VAR>;
@@ -560,27 +593,36 @@ stage_kernel(StageArgs<R> a) {
     // writes that region during the PML update, in operator 0's flux rows);
     // they are loaded together with the element id, so their round trip
     // overlaps that one instead of following the phase-1 batch.
-    R *sLast = S::FW ? sC : lds + S::OFF_F;   // [27][NP] during phase 1
-    static_assert(!PML || 27 * NP <= S::face_reals(EB), "last-element fluxes must fit the face region");
-    constexpr int NLS = PML ? (27 * NP + NTHR - 1) / NTHR : 1;
+    // Of the recomputing kernels stage 1 needs none, stage 2 those of both
+    // stages (FW shapes: the stage-1 ones in operator 2's flux rows).
+    constexpr bool LASTF = PML && RC != 1;
+    constexpr int NLASTF = RC == 2 ? 54 * NP : 27 * NP;
+    R *sLast = S::FW ? sC : lds + S::OFF_F;                     // [27][NP] during phase 1
+    R *sLast1 = S::FW ? sC + 24 * NT : lds + S::OFF_F + 27 * NP;  // [27][NP] stage-1 fluxes (RC 2)
+    static_assert(!LASTF || NLASTF <= S::face_reals(EB), "last-element fluxes must fit the face region");
+    static_assert(!S::FW || 27 * NP <= 9 * NT, "stage-1 fluxes must fit operator 2's flux rows");
+    constexpr int NLS = LASTF ? (NLASTF + NTHR - 1) / NTHR : 1;
     R lst[NLS];
-    if constexpr (PML) {
+    if constexpr (LASTF) {
         if (a.pml_compat) {
             const R *lastf = a.last_flux + (size_t)shot * 27 * NP;
+            const R *lastf1 = RC == 2 ? a.last_flux1 + (size_t)shot * 27 * NP : lastf;
 #pragma unroll
             for (int r = 0; r < NLS; ++r) {
                 const int i = t + r * NTHR;
-                lst[r] = lastf[i < 27 * NP ? i : 0];
+                if constexpr (RC == 2) lst[r] = *(i < 27 * NP ? lastf + i : lastf1 + (i < 54 * NP ? i - 27 * NP : 0));
+                else lst[r] = lastf[i < 27 * NP ? i : 0];
             }
         }
     }
     const int e = valid ? a.elist[idx] : 0;
-    if constexpr (PML) {
+    if constexpr (LASTF) {
         if (a.pml_compat) {
 #pragma unroll
             for (int r = 0; r < NLS; ++r) {
                 const int i = t + r * NTHR;
                 if (i < 27 * NP) sLast[i] = lst[r];
+                else if (i < NLASTF) sLast1[i - 27 * NP] = lst[r];
             }
         }
     }
@@ -591,7 +633,7 @@ stage_kernel(StageArgs<R> a) {
     // the RK base planes: stage 1 does not use the base (its weight is 0, or
     // A_1 = 0 for the low-storage residual), so their descriptors get size 0
     // there and the loads return 0 without touching memory
-    const unsigned pnb_base = a.irk == 1 ? 0u : pnb;
+    const unsigned pnb_base = RC != 2 && a.irk == 1 ? 0u : pnb;
     if (node_thr && j == 0) sElem[eb] = e;
     // the element's step (one value per element; the same for a whole mesh
     // unless instances of different steps share the launch)
@@ -675,7 +717,7 @@ stage_kernel(StageArgs<R> a) {
     R qs[9];
     R ef0 = 0, ef1 = 0, ef2 = 0, ef3 = 0, rho = 1;
     R qv[9], mv[9], m2 = 1, m3 = 0, m4 = 0;
-    R pc[PML ? 9 : 1], cur[PML ? 27 : 1], bse[PML ? 27 : 1];
+    R pc[PML ? 9 : 1], cur[PML ? 27 : 1], bse[PML && RC == 0 ? 27 : 1];
     const R *pin = a.pin + (size_t)shot * 27 * ng;
     const R *pbase = a.pbase + (size_t)shot * 27 * ng;
     R *pout = a.pout + (size_t)shot * 27 * ng;
@@ -696,11 +738,13 @@ stage_kernel(StageArgs<R> a) {
             for (int k = 0; k < 9; ++k) pc[k] = pload<BUF>(pmlc + k * ng, pnb, g32);
 #pragma unroll
             for (int c = 0; c < 27; ++c) cur[c] = pload<BUF>(pin + c * ng, pnb, g32);
+            if constexpr (RC == 0) {
 #pragma unroll
-            for (int c = 0; c < 27; ++c) bse[c] = pload<BUF>(pbase + c * ng, pnb_base, g32);
+                for (int c = 0; c < 27; ++c) bse[c] = pload<BUF>(pbase + c * ng, pnb_base, g32);
+            }
         }
     }
-    if constexpr (PML) __syncthreads();   // the staged fluxes are in LDS
+    if constexpr (LASTF) __syncthreads();   // the staged fluxes are in LDS
     // Node threads past the end of the list (last block only) carry element
     // 0's values through the node phases: finite, confined to their own
     // columns, never stored.
@@ -776,7 +820,7 @@ stage_kernel(StageArgs<R> a) {
             // stage-start values, so it is done here and the auxiliaries die
             R Fm[9], Gm[9], Hm[9];
             elastic_flux_node(qs, ef0, ef1, ef2, ef3, Fm, Gm, Hm);
-            const RkStage<R> rs = rk_stage<R>(a.scheme, a.irk, a.w13, a.w23, a.lsa, a.lsb);
+            const RkStage<R> rs = rk_stage<R, RC>(a.scheme, a.irk, a.w13, a.w23, a.lsa, a.lsb);
             // a shot whose PML is switched off (src/timeloopMod.f90:532-539)
             // keeps its PML elements in this launch with the modification
             // and the ADE update made neutral: auxiliaries read as 0,
@@ -799,7 +843,14 @@ stage_kernel(StageArgs<R> a) {
 #pragma unroll
                 for (int i = 0; i < 9; ++i) {
                     const int c = d * 9 + i;
-                    const R c0 = on ? cur[c] : R(0);
+                    R c0 = on ? cur[c] : R(0);
+                    if constexpr (RC == 2) {
+                        // the stage-1 value from the step-start one
+                        const R u1 = sLast1[c * NP + j];
+                        const R dadt1 = -al * c0 - dk * (c0 + u1);
+                        R none = 0;
+                        c0 = rk_update<R, false, false, 1>(rs, c0, none, dadt1, dt);
+                    }
                     const R mod = (c0 + FF[i]) * rk;
                     if constexpr (KC) {
 #pragma unroll
@@ -811,16 +862,18 @@ stage_kernel(StageArgs<R> a) {
                     } else if (i != skip) {
                         sX[(col++) * NT + t] = mod;
                     }
+                    if constexpr (RC == 1) continue;   // stage 2 repeats the update
                     // read unconditionally and selected (the region is
                     // stale without compat): no branch between components
                     const R lastv = sLast[c * NP + j];
-                    const R u = a.pml_compat ? lastv : mod;
+                    const R u = RC == 2 || a.pml_compat ? lastv : mod;
                     const R dadt = -al * c0 - dk * (c0 + u);
-                    pv[i] = rk_update<R, LS>(rs, c0, bse[c], dadt, dt);
+                    if constexpr (RC == 2) pv[i] = rk_update<R, false, false, 2>(rs, c0, cur[c], dadt, dt);
+                    else if constexpr (RC == 0) pv[i] = rk_update<R, LS>(rs, c0, bse[c], dadt, dt);
                 }
                 // one guarded block of stores per direction (a guard per
                 // store leaves waits for every earlier store at the joins)
-                if (valid) {
+                if (RC != 1 && valid) {
 #pragma unroll
                     for (int i = 0; i < 9; ++i) pstore<BUF>(pout + (d * 9 + i) * ng, pnb, g32, pv[i]);
                 }
@@ -1189,9 +1242,17 @@ stage_kernel(StageArgs<R> a) {
 
     // ---- assemble the right-hand side (node threads) -----------------------
     load_memory_variables();
-    R thb[ATT ? 18 : 1], qb[9];
+    R thb[ATT && RC == 0 ? 18 : 1], gr[ATT ? 6 : 1], qb[9];
     if (node_thr) {
-        if constexpr (ATT) {
+        if constexpr (ATT && RC == 2) {
+            const R *gin = a.rate_in + (size_t)shot * 6 * ng;
+#pragma unroll
+            for (int c = 0; c < 6; ++c) {
+                const R v = pload<BUF>(gin + c * ng, pnb, g32);
+                gr[c] = valid ? v : R(0);
+            }
+        }
+        if constexpr (ATT && RC == 0) {
             const R *thbase = a.thbase + (size_t)shot * 18 * ng;
             if (a.irk == 1) {
 #pragma unroll
@@ -1204,7 +1265,7 @@ stage_kernel(StageArgs<R> a) {
                 }
             }
         }
-        if (a.irk == 1) {
+        if (RC == 1 || (RC == 0 && a.irk == 1)) {
 #pragma unroll
             for (int f = 0; f < 9; ++f) qb[f] = qs[f];
         } else {
@@ -1275,12 +1336,24 @@ stage_kernel(StageArgs<R> a) {
                 exy = gv[3] + gv[1]; eyz = gv[7] + gv[5]; exz = gv[6] + gv[2];
             }
             R *thout = a.thout + (size_t)shot * 18 * ng;
-            const RkStage<R> rs = rk_stage<R>(a.scheme, a.irk, a.w13, a.w23, a.lsa, a.lsb);
+            const RkStage<R> rs = rk_stage<R, RC>(a.scheme, a.irk, a.w13, a.w23, a.lsa, a.lsb);
+            // the rates common to the mechanisms (recomputing kernels)
+            const R gn[6] = {lf[NFC - 6] - ex, lf[NFC - 5] - ey, lf[NFC - 4] - ez, lf[NFC - 3] - R(0.5) * exy,
+                             lf[NFC - 2] - R(0.5) * eyz, lf[NFC - 1] - R(0.5) * exz};
 #pragma unroll
             for (int i = 0; i < NMB; ++i) {
                 const R w = a.wl[i];
                 const R vol[6] = {-w * ex, -w * ey, -w * ez, R(-0.5) * w * exy, R(-0.5) * w * eyz, R(-0.5) * w * exz};
                 R *tm = th + i * 6;
+                R t0[6];
+                if constexpr (RC == 2) {
+#pragma unroll
+                    for (int c = 0; c < 6; ++c) {
+                        t0[c] = tm[c];
+                        R none = 0;
+                        tm[c] = rk_update<R, false, false, 1>(rs, t0[c], none, w * (gr[c] - t0[c]), dt);
+                    }
+                }
                 const R a1 = avc[i * 3 + 0], a2 = avc[i * 3 + 1], a3 = avc[i * 3 + 2];
                 rhs[0] = rhs[0] + a3 * tm[0] + a1 * (tm[1] + tm[2]);
                 rhs[1] = rhs[1] + a3 * tm[1] + a1 * (tm[2] + tm[0]);
@@ -1292,12 +1365,22 @@ stage_kernel(StageArgs<R> a) {
 #pragma unroll
                 for (int c = 0; c < 6; ++c) {
                     const int k = i * 6 + c;
-                    const R arq = vol[c] + w * lf[9 + c] - w * th[k];
-                    th[k] = rk_update<R, LS, sizeof(R) == 4>(rs, th[k], thb[k], arq, dt);
+                    if constexpr (RC == 2) {
+                        th[k] = rk_update<R, false, sizeof(R) == 4, 2>(rs, tm[c], t0[c], w * (gn[c] - tm[c]), dt);
+                    } else if constexpr (RC == 0) {
+                        const R arq = vol[c] + w * lf[9 + c] - w * th[k];
+                        th[k] = rk_update<R, LS, sizeof(R) == 4>(rs, th[k], thb[k], arq, dt);
+                    }
                 }
             }
             // one guarded block of stores
-            if (valid) {
+            if constexpr (RC == 1) {
+                R *gout = a.rate_out + (size_t)shot * 6 * ng;
+                if (valid) {
+#pragma unroll
+                    for (int c = 0; c < 6; ++c) pstore<BUF>(gout + c * ng, pnb, g32, gn[c]);
+                }
+            } else if (valid) {
 #pragma unroll
                 for (int k = 0; k < 18; ++k) pstore<BUF>(thout + k * ng, pnb, g32, th[k]);
             }
@@ -1351,20 +1434,24 @@ stage_kernel(StageArgs<R> a) {
             }
 #pragma unroll
             for (int f = 0; f < 9; ++f) {
-                const R v = pload<BUF>(a.qlo_base + so + f * ng, pnb_base, g32);
-                blo[f] = (a.irk == 1 || !valid) ? alo[f] : v;
+                if constexpr (RC == 1) {
+                    blo[f] = alo[f];
+                } else {
+                    const R v = pload<BUF>(a.qlo_base + so + f * ng, pnb_base, g32);
+                    blo[f] = ((RC == 0 && a.irk == 1) || !valid) ? alo[f] : v;
+                }
             }
 #pragma unroll
             for (int f = 0; f < 9; ++f) {
                 R lo;
-                rk_combine_comp<R>(a.scheme, a.irk, qs[f], alo[f], qb[f], blo[f], rhs[f], dt, a.w13, a.w23, qnew[f],
+                rk_combine_comp<R>(RC ? 2 : a.scheme, RC ? RC : a.irk, qs[f], alo[f], qb[f], blo[f], rhs[f], dt, a.w13, a.w23, qnew[f],
                                    lo);
                 if (valid) { pstore<BUF>(qout + f * ng, pnb, g32, qnew[f]); pstore<BUF>(a.qlo_out + so + f * ng, pnb, g32, lo); }
             }
         } else {
-            const RkStage<R> rs = rk_stage<R>(a.scheme, a.irk, a.w13, a.w23, a.lsa, a.lsb);
+            const RkStage<R> rs = rk_stage<R, RC>(a.scheme, a.irk, a.w13, a.w23, a.lsa, a.lsb);
 #pragma unroll
-            for (int f = 0; f < 9; ++f) qnew[f] = rk_update<R, LS, sizeof(R) == 4>(rs, qs[f], qb[f], rhs[f], dt);
+            for (int f = 0; f < 9; ++f) qnew[f] = rk_update<R, LS, sizeof(R) == 4, RC>(rs, qs[f], qb[f], rhs[f], dt);
             if (valid) {
 #pragma unroll
                 for (int f = 0; f < 9; ++f) pstore<BUF>(qout + f * ng, pnb, g32, qnew[f]);
@@ -1380,7 +1467,8 @@ stage_kernel(StageArgs<R> a) {
     }
 
     // ---- post-step (src/timeloopMod.f90:482-516) ---------------------------
-    if (a.last_stage) {
+    if (RC == 1) return;
+    if (RC == 2 || a.last_stage) {
         if (valid) {
             if (a.u_full) {
 #pragma unroll
@@ -1556,6 +1644,55 @@ __global__ void last_flux_kernel(const R *qin, const R *pin, const R *pmlc, cons
         out[(9 + i) * NP + j] = G[i];
         out[(18 + i) * NP + j] = H[i];
     }
+}
+
+// The same for the recomputing RK2 kernels, once per step between its stages:
+// out1 from the step-start state (q0, p0), out2 from the stage-1 state, whose
+// auxiliaries are formed from p0 as the stage kernel forms them.
+template <int ORDER, typename R>
+__global__ void last_flux_rk2_kernel(const R *q0, const R *q1, const R *p0, const R *pmlc, const R *matc, int last,
+                                     int last_is_pml, int nglob, int mat_stride, int pmlc_stride_ng, R dt0,
+                                     const R *dt_elem, R *out1, R *out2) {
+    constexpr int NP = Dims<ORDER>::NP;
+    const int j = threadIdx.x;
+    const int shot = blockIdx.x;
+    if (j >= NP) return;
+    const size_t ng = (size_t)nglob, g = (size_t)last * NP + j;
+    q0 += (size_t)shot * 9 * ng;
+    q1 += (size_t)shot * 9 * ng;
+    p0 += (size_t)shot * 27 * ng;
+    pmlc += (size_t)shot * pmlc_stride_ng * ng;
+    matc += (size_t)shot * mat_stride;
+    out1 += (size_t)shot * 27 * NP;
+    out2 += (size_t)shot * 27 * NP;
+    const R dt = dt_elem ? dt_elem[last] : dt0;
+    // every load first: one round trip
+    R qa[9], qb[9], p[27], pc[9];
+#pragma unroll
+    for (int f = 0; f < 9; ++f) { qa[f] = q0[f * ng + g]; qb[f] = q1[f * ng + g]; pc[f] = pmlc[f * ng + g]; }
+#pragma unroll
+    for (int c = 0; c < 27; ++c) p[c] = p0[c * ng + g];
+    const R *mc = matc + (size_t)last * 8;
+    const R lam = mc[3], mu = mc[4], rho = mc[2];
+    R F[3][9], E[3][9];
+    elastic_flux_node<R>(qa, -(lam + 2 * mu), -lam, -mu, R(-1.0) / rho, F[0], F[1], F[2]);
+    elastic_flux_node<R>(qb, -(lam + 2 * mu), -lam, -mu, R(-1.0) / rho, E[0], E[1], E[2]);
+    const RkStage<R> rs = rk_stage<R, 1>(2, 1, R(0), R(0), R(0), R(0));
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+#pragma unroll
+        for (int i = 0; i < 9; ++i) {
+            const int c = d * 9 + i;
+            R f1 = F[d][i], f2 = E[d][i];
+            if (last_is_pml) {
+                f1 = (p[c] + f1) / pc[6 + d];
+                const R dadt = -pc[d] * p[c] - pc[3 + d] * (p[c] + f1);
+                R none = 0;
+                f2 = (rk_update<R, false, false, 1>(rs, p[c], none, dadt, dt) + f2) / pc[6 + d];
+            }
+            out1[c * NP + j] = f1;
+            out2[c * NP + j] = f2;
+        }
 }
 
 // Receiver sampling (src/timeloopMod.f90:358-373) of row `row_offset + *d_it`

@@ -10,6 +10,17 @@ void launch_stage_one(const StageArgs<R> &a, hipStream_t s) {
     using S = Shape<ORDER, ATT, PML, R, VAR>;
     const unsigned grid = (unsigned)((a.nlist + S::EB - 1) / S::EB) * (unsigned)a.nshot;
     if (grid == 0) return;
+    if constexpr ((ATT || PML) && !LS) {
+        // the recomputing RK2 kernels (stage_kernel), chosen by the caller
+        if (a.recompute == 1) {
+            hipLaunchKernelGGL((stage_kernel<ORDER, ATT, PML, R, LS, VAR, 1>), dim3(grid), dim3(S::NTHR), 0, s, a);
+            return;
+        }
+        if (a.recompute == 2) {
+            hipLaunchKernelGGL((stage_kernel<ORDER, ATT, PML, R, LS, VAR, 2>), dim3(grid), dim3(S::NTHR), 0, s, a);
+            return;
+        }
+    }
     hipLaunchKernelGGL((stage_kernel<ORDER, ATT, PML, R, LS, VAR>), dim3(grid), dim3(S::NTHR), 0, s, a);
 }
 

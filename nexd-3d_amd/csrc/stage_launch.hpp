@@ -18,6 +18,13 @@ namespace nexd {
 template <typename R, bool LS, int VAR>
 void launch_stage(int order, bool att, bool pml, const StageArgs<R> &a, hipStream_t s);
 
+// Whether a run uses the recomputing RK2 kernels (stage_kernel, RC): TVD RK2
+// with memory variables or with PML auxiliaries whose update takes the last
+// element's fluxes (compat).
+constexpr bool recompute_rk2(int scheme, bool att, bool pml, bool pml_compat) {
+    return scheme == 2 && (att || pml) && (!pml || pml_compat);
+}
+
 // the block shapes the autotuner chooses from, for a real type and scheme
 template <typename R>
 constexpr int stage_variants(bool ls) { return (sizeof(R) == 4 && !ls) ? 2 : 1; }
