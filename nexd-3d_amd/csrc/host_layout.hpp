@@ -98,6 +98,48 @@ inline std::vector<double> mfma_lift_fragments(const std::vector<double> &LT, in
     return out;
 }
 
+// the nearest bfloat16 (finite values), its bits
+inline unsigned short bf16_bits(double x) {
+    const float f = (float)x;
+    unsigned u;
+    std::memcpy(&u, &f, 4);
+    u += 0x7fffu + ((u >> 16) & 1u);
+    return (unsigned short)(u >> 16);
+}
+inline double bf16_value(unsigned short b) {
+    const unsigned u = (unsigned)b << 16;
+    float f;
+    std::memcpy(&f, &u, 4);
+    return f;
+}
+
+// [Dr | Ds | Dt | LIFT] for the affine kernels, in the A-operand order of the
+// 16x16x32 BF16 MFMA, every entry as the sum of three bfloat16 (27 bits):
+// [step][row tile][part][lane][8].  Row tile rt holds nodes 16rt..16rt+15
+// (lane l: node 16rt + l%16).  The k index is dealt so that a lane of the B
+// operand supplies values of its own: entry i of step st is value s = 8 st + i
+// of lane group l/16, for s = 3 ks + o (ks < ceil(Np/4)) operator o at node
+// 4ks + l/16, then LIFT at face nodes 4ks + l/16; zero beyond Np and past the
+// last value.
+inline std::vector<unsigned short> mfma_affine_fragments(const std::vector<double> &D, const std::vector<double> &LT,
+                                                         int np, int nfp) {
+    const int nt = (np + 15) / 16, ksv = 3 * ((np + 3) / 4), kt = ksv + nfp / 4, ns = (kt + 7) / 8;
+    std::vector<unsigned short> out((size_t)ns * nt * 3 * 512, 0);
+    for (int s = 0; s < kt; ++s)
+        for (int rt = 0; rt < nt; ++rt)
+            for (int l = 0; l < 64; ++l) {
+                const int node = 16 * rt + l % 16, k = 4 * (s < ksv ? s / 3 : s - ksv) + l / 16;
+                if (node >= np || (s < ksv && k >= np)) continue;
+                double x = s < ksv ? D[((size_t)(s % 3) * np + node) * np + k] : LT[(size_t)k * np + node];
+                for (int p = 0; p < 3; ++p) {
+                    const unsigned short b = bf16_bits(x);
+                    out[((((size_t)(s / 8) * nt + rt) * 3 + p) * 64 + l) * 8 + s % 8] = b;
+                    x -= bf16_value(b);
+                }
+            }
+    return out;
+}
+
 // The mass matrix in the A-operand order of the 16x16x4 MFMA (the energy's
 // products M y): row tile mt holds nodes 16mt..16mt+15, k-step ks nodes
 // 4ks..4ks+3; lane l holds M(16mt + l%16, 4ks + l/16), zero beyond Np.  M is
@@ -178,6 +220,135 @@ inline std::string convert_mesh(int nelem, int np, int npf, const std::vector<in
         }
     }
     return "";
+}
+
+// inverse of a 3 x 3 matrix (row-major); false if it is singular
+inline bool invert3(const double *a, double *r) {
+    const double c0 = a[4] * a[8] - a[5] * a[7], c1 = a[5] * a[6] - a[3] * a[8], c2 = a[3] * a[7] - a[4] * a[6];
+    const double d = a[0] * c0 + a[1] * c1 + a[2] * c2, i = 1.0 / d;
+    r[0] = c0 * i; r[1] = (a[2] * a[7] - a[1] * a[8]) * i; r[2] = (a[1] * a[5] - a[2] * a[4]) * i;
+    r[3] = c1 * i; r[4] = (a[0] * a[8] - a[2] * a[6]) * i; r[5] = (a[2] * a[3] - a[0] * a[5]) * i;
+    r[6] = c2 * i; r[7] = (a[1] * a[6] - a[0] * a[7]) * i; r[8] = (a[0] * a[4] - a[1] * a[3]) * i;
+    return d != 0;
+}
+
+// The geometry of a straight-sided mesh, one set per element, for the affine
+// kernels.
+//
+// The Jacobian dx/d(r,s,t) of such an element is constant, but the reference
+// forms it with its Dr, Ds, Dt, whose rows differentiate a linear function to
+// about 1.5e-7 only (single-precision literals): J(i) = G (I + E(i)) at node i,
+// with E the same for every element, as the node coordinates are linear in r,
+// s, t.  Its derivatives are then
+//   sum_o M(i)_ok D_o f = sum_p Ginv_pk sum_o [(I + E(i))^-1]_op D_o f,   M = J^-1:
+// the constant metric Ginv with operators whose rows are combined once.  G is
+// the mean of J over the element's nodes, E comes from the first element.
+struct AffineHost {
+    std::vector<double> emet;    // [nelem][12] Ginv
+    std::vector<double> fgeo;    // [nelem][4][4] normal, half the mean face scale
+    std::vector<int> nbrt;       // [nelem][NFP] neighbour node, -1 free, -2 absorbing
+    std::vector<double> comb;    // [np][3][3] (I + E)^-1 of each node, rows o
+};
+
+// Whether the mesh is of that kind to single precision: every element's metric
+// is the first element's pattern times a constant, its face scales equal their
+// mean, and its face frames are orthonormal, each to 1e-6 (relative).  The
+// meshes of the host set-up are to 1e-12, 2e-7 and 2e-7.  Fills `o` if so.
+inline bool affine_mesh(const MeshHost &m, int nelem, int np, int npf, AffineHost &o) {
+    constexpr double tol = 1e-6;
+    const size_t ng = (size_t)nelem * np;
+    const int nfp = 4 * npf;
+    o.emet.assign((size_t)nelem * 12, 0.0);
+    o.fgeo.resize((size_t)nelem * 16);
+    o.nbrt.resize((size_t)nelem * nfp);
+    o.comb.assign((size_t)np * 9, 0.0);
+    std::vector<double> E((size_t)np * 9), C((size_t)np * 9);   // I + E and its inverse, [9][np]
+    {
+        std::vector<double> J((size_t)np * 9);
+        double G[9] = {0}, Gi[9], M[9], t[9];
+        for (int j = 0; j < np; ++j) {
+            for (int k = 0; k < 9; ++k) M[k] = m.metric[k * ng + j];
+            if (!invert3(M, &J[(size_t)j * 9])) return false;
+            for (int k = 0; k < 9; ++k) G[k] += J[(size_t)j * 9 + k] / np;
+        }
+        if (!invert3(G, Gi)) return false;
+        for (int j = 0; j < np; ++j) {
+            for (int r = 0; r < 3; ++r)
+                for (int q = 0; q < 3; ++q) {
+                    t[3 * r + q] = 0;
+                    for (int k = 0; k < 3; ++k) t[3 * r + q] += Gi[3 * r + k] * J[(size_t)j * 9 + 3 * k + q];
+                    E[(size_t)(3 * r + q) * np + j] = t[3 * r + q];
+                }
+            if (!invert3(t, &o.comb[(size_t)j * 9])) return false;
+            for (int k = 0; k < 9; ++k) C[(size_t)k * np + j] = o.comb[(size_t)j * 9 + k];
+        }
+    }
+    for (int e = 0; e < nelem; ++e) {
+        // Ginv: the mean of (I + E) M over the nodes, then M against (I + E)^-1 Ginv
+        const double *M = m.metric.data() + (size_t)e * np;
+        double Gi[9] = {0}, big = 0;
+        for (int r = 0; r < 3; ++r)
+            for (int k = 0; k < 3; ++k) {
+                double s0 = 0, s1 = 0, s2 = 0;
+                for (int j = 0; j < np; ++j) {
+                    s0 += E[(size_t)(3 * r) * np + j] * M[k * ng + j];
+                    s1 += E[(size_t)(3 * r + 1) * np + j] * M[(3 + k) * ng + j];
+                    s2 += E[(size_t)(3 * r + 2) * np + j] * M[(6 + k) * ng + j];
+                }
+                Gi[3 * r + k] = (s0 + s1 + s2) / np;
+            }
+        for (int k = 0; k < 9; ++k) {
+            const double b = Gi[k] < 0 ? -Gi[k] : Gi[k];
+            if (!(b <= big)) big = b;   // NaN stays and fails below
+        }
+        const double lim = tol * big;
+        int bad = !(big > 0);
+        for (int r = 0; r < 3; ++r)
+            for (int k = 0; k < 3; ++k) {
+                const double *t = M + (size_t)(3 * r + k) * ng, *c = &C[(size_t)3 * r * np];
+                for (int j = 0; j < np; ++j) {
+                    const double d = c[j] * Gi[k] + c[np + j] * Gi[3 + k] + c[2 * np + j] * Gi[6 + k] - t[j];
+                    bad |= !(d <= lim) | !(-d <= lim);
+                }
+            }
+        if (bad) return false;
+        for (int k = 0; k < 9; ++k) o.emet[(size_t)e * 12 + k] = Gi[k];
+        for (int f = 0; f < 4; ++f) {
+            const double *fs = m.fscale.data() + (size_t)e * nfp + f * npf, *fr = m.frame.data() + ((size_t)e * 4 + f) * 9;
+            double s = 0;
+            for (int i = 0; i < npf; ++i) s += fs[i];
+            s /= npf;
+            for (int i = 0; i < npf; ++i) {
+                const double d = fs[i] - s;
+                bad |= !(d <= tol * s) | !(-d <= tol * s);
+            }
+            for (int x = 0; x < 3; ++x)
+                for (int y = x; y < 3; ++y) {
+                    const double d = fr[3 * x] * fr[3 * y] + fr[3 * x + 1] * fr[3 * y + 1] + fr[3 * x + 2] * fr[3 * y + 2] -
+                                     (x == y ? 1.0 : 0.0);
+                    bad |= !(d <= tol) | !(-d <= tol);
+                }
+            double *g = o.fgeo.data() + ((size_t)e * 4 + f) * 4;
+            for (int k = 0; k < 3; ++k) g[k] = fr[k];
+            g[3] = 0.5 * s;
+            const int ft = m.ftype[(size_t)e * 4 + f];
+            const size_t at = (size_t)e * nfp + f * npf;
+            for (int i = 0; i < npf; ++i) o.nbrt[at + i] = ft >= 0 ? m.nbr[at + i] : ft;
+        }
+        if (bad) return false;
+    }
+    return true;
+}
+
+// the combined operators: row i of operator p is sum_o comb(i)_op D_o(i,:)
+inline std::vector<double> affine_operators(const std::vector<double> &D, int np, const std::vector<double> &comb) {
+    std::vector<double> out((size_t)3 * np * np, 0.0);
+    for (int p = 0; p < 3; ++p)
+        for (int i = 0; i < np; ++i)
+            for (int q = 0; q < 3; ++q)
+                for (int j = 0; j < np; ++j)
+                    out[((size_t)p * np + i) * np + j] += comb[(size_t)i * 9 + 3 * q + p] * D[((size_t)q * np + i) * np + j];
+    return out;
 }
 
 inline void pml_coefficients(size_t ng, const double *ddx, const double *ddy, const double *ddz,

@@ -54,6 +54,12 @@ struct Batch : BatchBase {
     R *paux[2] = {nullptr, nullptr};
     R *D = nullptr, *DK = nullptr, *LT = nullptr, *mass = nullptr, *metric = nullptr, *fscale = nullptr, *frame = nullptr;
     R *jac = nullptr;
+    unsigned short *AK = nullptr;                        // affine kernels (straight-sided meshes, FP32)
+    R *emet = nullptr, *fgeo = nullptr;
+    int *nbrt = nullptr;
+    bool affine = false;
+    nexd::OpsHost ops_host;
+    std::vector<double> affine_comb;   // AffineHost::comb of the mesh
     int *fmask = nullptr, *nbr = nullptr, *ftype = nullptr;
     std::vector<int> fmask_host;
     R *matc = nullptr, *anel = nullptr, *pmlc = nullptr, *emat = nullptr;
@@ -191,6 +197,10 @@ struct Batch : BatchBase {
 
     // element blocks of one list launch (per shot)
     int nblocks(int n, bool pml) const {
+        if (affine) {
+            const int eb = nexd::affine_eb(cfg.order, cfg.attenuation != 0, pml, tile);
+            return (n + eb - 1) / eb;
+        }
         return nexd::stage_blocks<R>(cfg.order, n, cfg.attenuation != 0, pml, tile);
     }
 
@@ -203,12 +213,20 @@ struct Batch : BatchBase {
         int rc;
         if (n_plain && (rc = put(elist_plain, plain))) return rc;
         if (n_pml && (rc = put(elist_pml, pmll))) return rc;
-        nblk_total = nblocks(n_plain, false) + nblocks(n_pml, true);
+        count_blocks();
         drop_graph();
         return 0;
     }
 
-    using TileKey = std::tuple<int, int, int, int, int, int, int, int>;
+    // the affine kernels' operators, from the uploaded ones and the mesh
+    int put_affine_operators() {
+        return upload(&AK, nexd::mfma_affine_fragments(nexd::affine_operators(ops_host.D, np, affine_comb), ops_host.LT, np,
+                                                       4 * npf));
+    }
+
+    void count_blocks() { nblk_total = nblocks(n_plain, false) + nblocks(n_pml, true); }
+
+    using TileKey = std::tuple<int, int, int, int, int, int, int, int, bool>;
     static std::map<TileKey, std::pair<int, std::vector<double>>> &tile_cache() {
         static std::map<TileKey, std::pair<int, std::vector<double>>> c;
         return c;
@@ -264,12 +282,20 @@ struct Batch : BatchBase {
         a.mass = mass; a.jac = jac; a.emat = emat;
         a.emat_stride = cfg.shared_material ? 0 : cfg.nelem * 2;
         a.pml_on = cfg.pml ? pml_on : nullptr;
+        a.AK = AK; a.emet = emet; a.fgeo = fgeo; a.nbrt = nbrt;
         return a;
     }
 
     void dispatch(const nexd::StageArgs<R> &a, bool pml) { dispatch(a, pml, stream); }
     void dispatch(const nexd::StageArgs<R> &a, bool pml, hipStream_t s) {
         const bool att = cfg.attenuation != 0;
+        if constexpr (sizeof(R) == 4) {
+            if (affine) {
+                if (tile == 1) nexd::launch_affine<1>(cfg.order, att, pml, a, s);
+                else nexd::launch_affine<0>(cfg.order, att, pml, a, s);
+                return;
+            }
+        }
         if (a.scheme == NEXD_LSRK4) {
             nexd::launch_stage<R, true, 0>(cfg.order, att, pml, a, s);
         } else if (tile == 1) {
@@ -284,7 +310,7 @@ struct Batch : BatchBase {
     int set_tile(int t) {
         if (t < 0 || t >= nvariants()) return fail(NEXD_E_ARG, "no such block shape for this precision and scheme");
         tile = t;
-        nblk_total = nblocks(n_plain, false) + nblocks(n_pml, true);
+        count_blocks();
         drop_graph();
         return 0;
     }
@@ -292,13 +318,13 @@ struct Batch : BatchBase {
     // Times every block shape on this batch's own element lists (one round
     // of all RK stages per list, nrep rounds after a warm-up) and keeps the
     // fastest.  Choices are remembered per (order, attenuation, PML,
-    // precision, shots, elements, PML elements) for the process, so
+    // precision, shots, elements, PML elements, kernel) for the process, so
     // batches of the same kind reuse them without timing.  The timing
     // overwrites the state: the batch is reset afterwards.
     int autotune(int nrep, int *choice, double *ms_out) {
         const int nv = nvariants();
         const auto key = std::make_tuple(cfg.order, cfg.attenuation, cfg.pml, cfg.precision, cfg.nshot, cfg.nelem,
-                                         n_pml, cfg.timeint * 2 + (cfg.compensated ? 1 : 0));
+                                         n_pml, cfg.timeint * 2 + (cfg.compensated ? 1 : 0), affine);
         std::vector<double> ms(nv, 0.0);
         int best = 0;
         auto &cache = tile_cache();
@@ -630,6 +656,8 @@ int upload_ops(Batch<R> *b, const double *dr, const double *ds, const double *dt
         (rc = b->upload(&b->mass, cvt<R>(nexd::mfma_mass_fragments(o.M, b->np)))) || (rc = b->upload(&b->fmask, o.fm)))
         return rc;
     b->fmask_host = o.fm;
+    b->ops_host = o;
+    if (b->affine && (rc = b->put_affine_operators())) return rc;
     b->have_ops = true;
     b->drop_graph();
     return 0;
@@ -646,11 +674,25 @@ int upload_mesh(Batch<R> *b, const int *ibool, const double *const met[9], const
     if (!err.empty())
         return err[0] == '!' ? b->fail(NEXD_E_UNSUPPORTED, err.substr(1)) : b->fail(NEXD_E_ARG, err);
     int rc;
-    if ((rc = b->upload(&b->metric, cvt<R>(m.metric))) || (rc = b->upload(&b->jac, cvt<R>(m.jac))) ||
-        (rc = b->upload(&b->fscale, cvt<R>(m.fscale))) || (rc = b->upload(&b->frame, cvt<R>(m.frame))) ||
-        (rc = b->upload(&b->nbr, m.nbr)) || (rc = b->upload(&b->ftype, m.ftype)))
+    // straight-sided meshes take the affine kernels in FP32 (TVD schemes, order
+    // 2 and up), every other the general ones
+    nexd::AffineHost ah;
+    const bool affine = sizeof(R) == 4 && b->cfg.timeint != NEXD_LSRK4 && b->cfg.order >= nexd::kAffMinOrder &&
+                        nexd::affine_mesh(m, b->cfg.nelem, b->np, b->npf, ah);
+    if ((rc = b->upload(&b->jac, cvt<R>(m.jac)))) return rc;
+    if (affine) {
+        b->affine_comb = ah.comb;
+        if ((rc = b->put_affine_operators()) || (rc = b->upload(&b->emet, cvt<R>(ah.emet))) ||
+            (rc = b->upload(&b->fgeo, cvt<R>(ah.fgeo))) || (rc = b->upload(&b->nbrt, ah.nbrt)))
+            return rc;
+    } else if ((rc = b->upload(&b->metric, cvt<R>(m.metric))) || (rc = b->upload(&b->fscale, cvt<R>(m.fscale))) ||
+               (rc = b->upload(&b->frame, cvt<R>(m.frame))) || (rc = b->upload(&b->nbr, m.nbr)) ||
+               (rc = b->upload(&b->ftype, m.ftype))) {
         return rc;
+    }
+    b->affine = affine;
     b->have_mesh = true;
+    b->count_blocks();
     b->drop_graph();
     return 0;
 }
@@ -667,6 +709,7 @@ int upload_material(Batch<R> *b, int shot, const double *vpu, const double *vsu,
         if (!(rho[e] > 0)) return b->fail(NEXD_E_ARG, "density must be positive");
         mc[e * 8 + 0] = (R)vpu[e]; mc[e * 8 + 1] = (R)vsu[e]; mc[e * 8 + 2] = (R)rho[e];
         mc[e * 8 + 3] = (R)lambdau[e]; mc[e * 8 + 4] = (R)muu[e];
+        mc[e * 8 + 5] = (R)(lambdau[e] * vpu[e] / (lambdau[e] + 2 * muu[e])); mc[e * 8 + 6] = (R)(1.0 / rho[e]);
         em[e * 2] = (R)mu[e]; em[e * 2 + 1] = (R)lambda[e];
     }
     if ((rc = b->put(b->matc + (size_t)shot * nel * 8, mc)) || (rc = b->put(b->emat + (size_t)shot * nel * 2, em)))

@@ -535,6 +535,7 @@ int nexd_upload_material(nexd_ctx *c, const double *vpu, const double *vsu, cons
         if (!(rho[e] > 0)) return fail(c, NEXD_E_ARG, "density must be positive");
         mc[e * 8 + 0] = vpu[e]; mc[e * 8 + 1] = vsu[e]; mc[e * 8 + 2] = rho[e];
         mc[e * 8 + 3] = lambdau[e]; mc[e * 8 + 4] = muu[e];
+        mc[e * 8 + 5] = lambdau[e] * vpu[e] / (lambdau[e] + 2 * muu[e]); mc[e * 8 + 6] = 1.0 / rho[e];
         em[e * 2] = mu[e]; em[e * 2 + 1] = lambda[e];
     }
     int rc;

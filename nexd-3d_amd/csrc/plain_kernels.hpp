@@ -81,7 +81,7 @@ struct StageArgs {
     const R *metric;            // [9][nglob] rx ry rz sx sy sz tx ty tz
     const R *fscale;            // [nelem][NFP]
     const R *frame;             // [nelem][4][9] n s t
-    const R *matc;              // [nelem][8] vp vs rho lam mu
+    const R *matc;              // [nelem][8] vp vs rho lam mu, lam vp/(lam+2mu), 1/rho
     const int *nbr;             // [nelem][4][NPF] neighbour node or -1
     const int *ftype;           // [nelem][4] >=0 interior, -1 free, -2 absorbing
     const R *anel;              // [nelem][NMB][3]
@@ -108,6 +108,11 @@ struct StageArgs {
     const R *emat;              // [nelem][2] mu, lambda for the energy
     int emat_stride;            // per-shot stride of emat (0: shared)
     const int *pml_on;          // [shot] 0 once a shot's PML is switched off; null: on
+    // the affine kernels' operands (affine_kernels.hpp), FP32
+    const unsigned short *AK;   // [Dr|Ds|Dt|LIFT] in three bfloat16 parts [step][row tile][part][64][8]
+    const R *emet;              // [nelem][12] metric (9) and padding
+    const R *fgeo;              // [nelem][4][4] normal, half the face scale
+    const int *nbrt;            // [nelem][4][NPF] neighbour node, -1 free, -2 absorbing
     // compensated state (float pairs hi + lo for the 9 wavefield components
     // and the receiver-element displacement); null when not compensated
     const R *qlo_in;            // [9][nglob] low parts of qin
@@ -513,6 +518,170 @@ struct Mfma<double> {
     }
 };
 
+// sources of node j's element (src/timeloopMod.f90:467-475): a list starting
+// at `first`, added to the node's right-hand side
+template <int NP, typename R>
+__device__ __forceinline__ void add_sources(const StageArgs<R> &a, int shot, int j, int first, int it_step, R rhs[9]) {
+    const int *next = a.src_next + (size_t)shot * a.nsrc;
+    const int *stype = a.srctype + (size_t)shot * a.nsrc;
+    for (int s = first; s >= 0; s = next[s]) {
+        if (a.src_factored) {
+            // spatial operand times the source time function of the step
+            const R *sp = a.src_spatial + (((size_t)shot * a.nsrc + s) * 6) * NP + j;
+            const R amp = a.src_stf[((size_t)shot * a.nsrc + s) * a.nt + it_step];
+            if (stype[s] == 0) {
+                rhs[6] += sp[0] * amp; rhs[7] += sp[NP] * amp; rhs[8] += sp[2 * NP] * amp;
+            } else {
+#pragma unroll
+                for (int c = 0; c < 6; ++c) rhs[c] += sp[c * NP] * amp;
+            }
+        } else if (stype[s] == 0) {
+            const R *sp = a.src_array + (((size_t)it_step * a.nsrc + s) * 3) * NP + j;
+            rhs[6] += sp[0]; rhs[7] += sp[NP]; rhs[8] += sp[2 * NP];
+        } else {
+            const R *sp = a.src_array_m + (((size_t)it_step * a.nsrc + s) * 6) * NP + j;
+#pragma unroll
+            for (int c = 0; c < 6; ++c) rhs[c] += sp[c * NP];
+        }
+    }
+}
+
+// displacement (forward Euler, compensated by Kahan's sum where low parts are
+// kept) and acceleration of a receiver element's node after a step
+template <int NP, typename R>
+__device__ __forceinline__ void update_receiver(const StageArgs<R> &a, int shot, int j, int slot, R dt, const R qnew[9],
+                                                const R rhs[9]) {
+    const size_t so = (size_t)shot * a.nslot + slot;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        R *u = a.u_slot + (so * 3 + c) * NP + j;
+        if (a.u_slot_lo) {
+            R *ul = a.u_slot_lo + (so * 3 + c) * NP + j;
+            R s, e;
+            two_sum(*u, dt * qnew[6 + c], s, e);
+            fast_two_sum(s, e + *ul, *u, *ul);
+        } else {
+            *u = *u + dt * qnew[6 + c];
+        }
+        a.a_slot[(so * 3 + c) * NP + j] = rhs[6 + c];
+    }
+}
+
+// Energy partial of a block (src/timeloopMod.f90:490-516), summed
+// in FP64.  Per element e and field pair: sum over nodes of
+// x . (M y), with y the velocities and the reference's strain
+// columns and x the velocities and stresses.  The products M y run
+// on the matrix cores: M (node tiles of 16, k-steps of 4 nodes,
+// fragments from a.mass) times the block's EB*9 columns y, one
+// column per lane; each lane then dots its column with x and
+// scales by its element's coefficient.  The reference's normal
+// "strains" are stress combinations divided by temp1 = 1/(4 mu^2 +
+// 6 mu lam), that is multiplied by ce = 4 mu^2 + 6 mu lam; with
+// stresses of a few 1e10 the products leave the FP32 range, so FP32
+// carries the combinations through the mass product and applies
+// ce in FP64.  FP64 follows the reference.
+// lds: 24 * EB * NP + 4 * EB reals, free for use after a barrier.
+template <int ORDER, int EB, int NTHR, typename R>
+__device__ __forceinline__ void block_energy(const StageArgs<R> &a, R *lds, int shot, int eblk, bool node_thr, bool valid,
+                                             int t, int eb, int j, int e, R rho, const R qnew[9]) {
+    constexpr int NP = Dims<ORDER>::NP, NT = EB * NP;
+    constexpr bool F32 = sizeof(R) == 4;
+    constexpr int NKE = (NP + 3) / 4, MTE = (NP + 15) / 16;   // k-steps, node tiles of M
+    constexpr int NCE = EB * 9, CTE = (NCE + 15) / 16;          // columns, column tiles
+    __syncthreads();
+    R *sE = lds;                  // [15][NT] y (rows 6..14 are the columns' values)
+    R *sX = lds + 15 * NT;        // [9][NT]  x = q after the step
+    R *sEl = lds + 24 * NT;       // [EB][4]  rho, mu, lambda, J of each element
+    if (node_thr) {
+        R lam_e = 0, mu_e = 0;
+        if (valid) {
+            const R *em = a.emat + (size_t)shot * a.emat_stride + (size_t)e * 2;
+            mu_e = em[0]; lam_e = em[1];
+        }
+        const R temp1 = R(1.) / (4 * mu_e * mu_e + 6 * mu_e * lam_e);
+        const R temp2 = 2 * mu_e;
+        R y[15];
+#pragma unroll
+        for (int c = 0; c < 9; ++c) y[c] = qnew[c];
+        const R c0 = 2 * (lam_e + mu_e) * qnew[0] - lam_e * (qnew[1] + qnew[2]);
+        const R c1 = 2 * (lam_e + mu_e) * qnew[1] - lam_e * (qnew[0] + qnew[2]);
+        const R c2 = 2 * (lam_e + mu_e) * qnew[2] - lam_e * (qnew[0] + qnew[0]);
+        y[9] = F32 ? c0 : c0 / temp1;
+        y[10] = F32 ? c1 : c1 / temp1;
+        y[11] = F32 ? c2 : c2 / temp1;
+        y[12] = qnew[3] / temp2; y[13] = qnew[4] / temp2; y[14] = qnew[5] / temp2;
+#pragma unroll
+        for (int c = 6; c < 15; ++c) sE[c * NT + t] = valid ? y[c] : R(0);
+#pragma unroll
+        for (int c = 0; c < 9; ++c) sX[c * NT + t] = valid ? qnew[c] : R(0);
+        if (j == 0) {
+            R *el = sEl + eb * 4;
+            el[0] = valid ? rho : R(0);
+            el[1] = mu_e;
+            el[2] = lam_e;
+            el[3] = valid ? a.jac[(size_t)e * NP] : R(0);
+        }
+    }
+    __syncthreads();
+    double part = 0;
+    {
+        using V4 = typename Mfma<R>::v4;
+        constexpr int NWE = NTHR / 64, CPWE = (CTE + NWE - 1) / NWE;   // column tiles per wave
+        const int lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+#pragma unroll
+        for (int cw = 0; cw < CPWE; ++cw) {
+            const int ct = w + cw * NWE;
+            if (ct >= CTE) break;
+            // column kind 0..2: velocities (x = v, y = v), 3..5: normal
+            // (x = sigma_ii, y = strain combination), 6..8: shear
+            const int col = ct * 16 + (lane & 15);
+            const bool cok = col < NCE;
+            const int ce = cok ? col / 9 : 0, kind = cok ? col - (col / 9) * 9 : 0;
+            const int xr = kind < 3 ? 6 + kind : kind - 3;
+            const R *yc = sE + (6 + kind) * NT + ce * NP;
+            const R *xc = sX + xr * NT + ce * NP;
+            R bfr[NKE];
+#pragma unroll
+            for (int ks = 0; ks < NKE; ++ks) {
+                const int m = 4 * ks + (lane >> 4);
+                bfr[ks] = yc[m < NP ? m : 0];   // M is zero beyond Np
+            }
+            double dsum = 0;
+#pragma unroll
+            for (int mt = 0; mt < MTE; ++mt) {
+                R afr[NKE];
+#pragma unroll
+                for (int ks = 0; ks < NKE; ++ks) afr[ks] = a.mass[(mt * NKE + ks) * 64 + lane];
+                V4 acc = {0, 0, 0, 0};
+#pragma unroll
+                for (int ks = 0; ks < NKE; ++ks) acc = Mfma<R>::fma(afr[ks], bfr[ks], acc);
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const int node = mt * 16 + (sizeof(R) == 8 ? 4 * v + (lane >> 4) : 4 * (lane >> 4) + v);
+                    if (node < NP) dsum += (double)(xc[node] * acc[v]);
+                }
+            }
+            const R *el = sEl + ce * 4;
+            const double mu = el[1], lam = el[2];
+            const double coef = kind < 3 ? (double)el[0] : (kind < 6 ? (F32 ? 4 * mu * mu + 6 * mu * lam : 1.0)
+                                                                       : 2.0);
+            part += cok ? 0.5 * (double)el[3] * coef * dsum : 0.0;
+        }
+    }
+    // block sum in a fixed order: within each wave, then over the waves
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) part += __shfl_down(part, off, 64);
+    __shared__ double sWave[NTHR / 64];
+    if ((t & 63) == 0) sWave[t >> 6] = part;
+    __syncthreads();
+    if (t == 0) {
+        double sum = 0;
+#pragma unroll
+        for (int i = 0; i < NTHR / 64; ++i) sum += sWave[i];
+        a.blk_energy[(size_t)shot * a.blk_stride + eblk] = sum;
+    }
+}
+
 // LS: the low-storage RK4 instantiation (residuals read and written in
 // place of the RK base); the TVD schemes use LS = false.  VAR: the block
 // shape (Shape).
@@ -562,6 +731,7 @@ stage_kernel(StageArgs<R> a) {
     R *sM = lds + S::OFF_M;               // [9][NT]     metric of the block's nodes
     R *sL = lds + S::OFF_L;               // [16][SLN]   lifted face values, node rows
     static_assert(NTHR % 64 == 0, "the energy block sum assumes whole waves");
+    static_assert(24 * NT + 4 * EB <= S::LDS, "energy values must fit the LDS");
 
     const int t = threadIdx.x;
     const size_t ng = (size_t)a.nglob;
@@ -1398,31 +1568,7 @@ stage_kernel(StageArgs<R> a) {
     if (node_thr) {
 #pragma unroll
         for (int f = 0; f < 9; ++f) rhs[f] = rhs[f] + lf[f];
-        // sources (src/timeloopMod.f90:467-475)
-        if (valid) {
-            const int *next = a.src_next + (size_t)shot * a.nsrc;
-            const int *stype = a.srctype + (size_t)shot * a.nsrc;
-            for (int s = src_first; s >= 0; s = next[s]) {
-                if (a.src_factored) {
-                    // spatial operand times the source time function of the step
-                    const R *sp = a.src_spatial + (((size_t)shot * a.nsrc + s) * 6) * NP + j;
-                    const R amp = a.src_stf[((size_t)shot * a.nsrc + s) * a.nt + it_step];
-                    if (stype[s] == 0) {
-                        rhs[6] += sp[0] * amp; rhs[7] += sp[NP] * amp; rhs[8] += sp[2 * NP] * amp;
-                    } else {
-#pragma unroll
-                        for (int c = 0; c < 6; ++c) rhs[c] += sp[c * NP] * amp;
-                    }
-                } else if (stype[s] == 0) {
-                    const R *sp = a.src_array + (((size_t)it_step * a.nsrc + s) * 3) * NP + j;
-                    rhs[6] += sp[0]; rhs[7] += sp[NP]; rhs[8] += sp[2 * NP];
-                } else {
-                    const R *sp = a.src_array_m + (((size_t)it_step * a.nsrc + s) * 6) * NP + j;
-#pragma unroll
-                    for (int c = 0; c < 6; ++c) rhs[c] += sp[c * NP];
-                }
-            }
-        }
+        if (valid) add_sources<NP>(a, shot, j, src_first, it_step, rhs);
         // Runge-Kutta update
         if (!LS && a.qlo_out) {
             const size_t so = (size_t)shot * 9 * ng;
@@ -1474,136 +1620,9 @@ stage_kernel(StageArgs<R> a) {
 #pragma unroll
                 for (int c = 0; c < 3; ++c) a.u_full[c * ng + g] = a.u_full[c * ng + g] + dt * qnew[6 + c];
             }
-            const int slot = rec_slot_e;
-            if (slot >= 0) {
-                const size_t so = (size_t)shot * a.nslot + slot;
-#pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    R *u = a.u_slot + (so * 3 + c) * NP + j;
-                    if (a.u_slot_lo) {
-                        // displacement by forward Euler, compensated (Kahan)
-                        R *ul = a.u_slot_lo + (so * 3 + c) * NP + j;
-                        R s, e;
-                        two_sum(*u, dt * qnew[6 + c], s, e);
-                        fast_two_sum(s, e + *ul, *u, *ul);
-                    } else {
-                        *u = *u + dt * qnew[6 + c];
-                    }
-                    a.a_slot[(so * 3 + c) * NP + j] = rhs[6 + c];
-                }
-            }
+            if (rec_slot_e >= 0) update_receiver<NP>(a, shot, j, rec_slot_e, dt, qnew, rhs);
         }
-        if (a.blk_energy) {
-            // energy partial of this block (src/timeloopMod.f90:490-516), summed
-            // in FP64.  Per element e and field pair: sum over nodes of
-            // x . (M y), with y the velocities and the reference's strain
-            // columns and x the velocities and stresses.  The products M y run
-            // on the matrix cores: M (node tiles of 16, k-steps of 4 nodes,
-            // fragments from a.mass) times the block's EB*9 columns y, one
-            // column per lane; each lane then dots its column with x and
-            // scales by its element's coefficient.  The reference's normal
-            // "strains" are stress combinations divided by temp1 = 1/(4 mu^2 +
-            // 6 mu lam), that is multiplied by ce = 4 mu^2 + 6 mu lam; with
-            // stresses of a few 1e10 the products leave the FP32 range, so FP32
-            // carries the combinations through the mass product and applies
-            // ce in FP64.  FP64 follows the reference.
-            constexpr bool F32 = sizeof(R) == 4;
-            constexpr int NKE = (NP + 3) / 4, MTE = (NP + 15) / 16;   // k-steps, node tiles of M
-            constexpr int NCE = EB * 9, CTE = (NCE + 15) / 16;          // columns, column tiles
-            __syncthreads();
-            R *sE = lds;                  // [15][NT] y (rows 6..14 are the columns' values)
-            R *sX = lds + 15 * NT;        // [9][NT]  x = q after the step
-            R *sEl = lds + 24 * NT;       // [EB][4]  rho, mu, lambda, J of each element
-            static_assert(24 * NT + 4 * EB <= S::LDS, "energy values must fit the LDS");
-            if (node_thr) {
-                R lam_e = 0, mu_e = 0;
-                if (valid) {
-                    const R *em = a.emat + (size_t)shot * a.emat_stride + (size_t)e * 2;
-                    mu_e = em[0]; lam_e = em[1];
-                }
-                const R temp1 = R(1.) / (4 * mu_e * mu_e + 6 * mu_e * lam_e);
-                const R temp2 = 2 * mu_e;
-                R y[15];
-#pragma unroll
-                for (int c = 0; c < 9; ++c) y[c] = qnew[c];
-                const R c0 = 2 * (lam_e + mu_e) * qnew[0] - lam_e * (qnew[1] + qnew[2]);
-                const R c1 = 2 * (lam_e + mu_e) * qnew[1] - lam_e * (qnew[0] + qnew[2]);
-                const R c2 = 2 * (lam_e + mu_e) * qnew[2] - lam_e * (qnew[0] + qnew[0]);
-                y[9] = F32 ? c0 : c0 / temp1;
-                y[10] = F32 ? c1 : c1 / temp1;
-                y[11] = F32 ? c2 : c2 / temp1;
-                y[12] = qnew[3] / temp2; y[13] = qnew[4] / temp2; y[14] = qnew[5] / temp2;
-#pragma unroll
-                for (int c = 6; c < 15; ++c) sE[c * NT + t] = valid ? y[c] : R(0);
-#pragma unroll
-                for (int c = 0; c < 9; ++c) sX[c * NT + t] = valid ? qnew[c] : R(0);
-                if (j == 0) {
-                    R *el = sEl + eb * 4;
-                    el[0] = valid ? rho : R(0);
-                    el[1] = mu_e;
-                    el[2] = lam_e;
-                    el[3] = valid ? a.jac[(size_t)e * NP] : R(0);
-                }
-            }
-            __syncthreads();
-            double part = 0;
-            {
-                using V4 = typename Mfma<R>::v4;
-                constexpr int NWE = NTHR / 64, CPWE = (CTE + NWE - 1) / NWE;   // column tiles per wave
-                const int lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
-#pragma unroll
-                for (int cw = 0; cw < CPWE; ++cw) {
-                    const int ct = w + cw * NWE;
-                    if (ct >= CTE) break;
-                    // column kind 0..2: velocities (x = v, y = v), 3..5: normal
-                    // (x = sigma_ii, y = strain combination), 6..8: shear
-                    const int col = ct * 16 + (lane & 15);
-                    const bool cok = col < NCE;
-                    const int ce = cok ? col / 9 : 0, kind = cok ? col - (col / 9) * 9 : 0;
-                    const int xr = kind < 3 ? 6 + kind : kind - 3;
-                    const R *yc = sE + (6 + kind) * NT + ce * NP;
-                    const R *xc = sX + xr * NT + ce * NP;
-                    R bfr[NKE];
-#pragma unroll
-                    for (int ks = 0; ks < NKE; ++ks) {
-                        const int m = 4 * ks + (lane >> 4);
-                        bfr[ks] = yc[m < NP ? m : 0];   // M is zero beyond Np
-                    }
-                    double dsum = 0;
-#pragma unroll
-                    for (int mt = 0; mt < MTE; ++mt) {
-                        R afr[NKE];
-#pragma unroll
-                        for (int ks = 0; ks < NKE; ++ks) afr[ks] = a.mass[(mt * NKE + ks) * 64 + lane];
-                        V4 acc = {0, 0, 0, 0};
-#pragma unroll
-                        for (int ks = 0; ks < NKE; ++ks) acc = Mfma<R>::fma(afr[ks], bfr[ks], acc);
-#pragma unroll
-                        for (int v = 0; v < 4; ++v) {
-                            const int node = mt * 16 + (sizeof(R) == 8 ? 4 * v + (lane >> 4) : 4 * (lane >> 4) + v);
-                            if (node < NP) dsum += (double)(xc[node] * acc[v]);
-                        }
-                    }
-                    const R *el = sEl + ce * 4;
-                    const double mu = el[1], lam = el[2];
-                    const double coef = kind < 3 ? (double)el[0] : (kind < 6 ? (F32 ? 4 * mu * mu + 6 * mu * lam : 1.0)
-                                                                               : 2.0);
-                    part += cok ? 0.5 * (double)el[3] * coef * dsum : 0.0;
-                }
-            }
-            // block sum in a fixed order: within each wave, then over the waves
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1) part += __shfl_down(part, off, 64);
-            __shared__ double sWave[NTHR / 64];
-            if ((t & 63) == 0) sWave[t >> 6] = part;
-            __syncthreads();
-            if (t == 0) {
-                double sum = 0;
-#pragma unroll
-                for (int i = 0; i < NTHR / 64; ++i) sum += sWave[i];
-                a.blk_energy[(size_t)shot * a.blk_stride + eblk] = sum;
-            }
-        }
+        if (a.blk_energy) block_energy<ORDER, EB, NTHR>(a, lds, shot, eblk, node_thr, valid, t, eb, j, e, rho, qnew);
     }
 }
 

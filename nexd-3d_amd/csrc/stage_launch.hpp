@@ -7,6 +7,7 @@
 
 #include <type_traits>
 
+#include "affine_kernels.hpp"
 #include "plain_kernels.hpp"
 
 namespace nexd {
@@ -18,6 +19,13 @@ namespace nexd {
 template <typename R, bool LS, int VAR>
 void launch_stage(int order, bool att, bool pml, const StageArgs<R> &a, hipStream_t s);
 
+constexpr int kAffMinOrder = 2;
+
+// Launches affine_kernel<order, att, pml, VAR> (FP32, TVD schemes, straight-
+// sided meshes) for a.nlist elements and a.nshot shots on stream s.
+template <int VAR>
+void launch_affine(int order, bool att, bool pml, const StageArgs<float> &a, hipStream_t s);
+
 // Whether a run uses the recomputing RK2 kernels (stage_kernel, RC): TVD RK2
 // with memory variables or with PML auxiliaries whose update takes the last
 // element's fluxes (compat).
@@ -28,6 +36,27 @@ constexpr bool recompute_rk2(int scheme, bool att, bool pml, bool pml_compat) {
 // the block shapes the autotuner chooses from, for a real type and scheme
 template <typename R>
 constexpr int stage_variants(bool ls) { return (sizeof(R) == 4 && !ls) ? 2 : 1; }
+
+// elements per block of an affine kernel
+inline int affine_eb(int order, bool att, bool pml, int var) {
+    auto pick = [&](auto ord) {
+        constexpr int O = decltype(ord)::value;
+        auto shape = [&](auto v) {
+            constexpr int V = decltype(v)::value;
+            if (att && pml) return AffShape<O, true, true, V>::EB;
+            if (att) return AffShape<O, true, false, V>::EB;
+            if (pml) return AffShape<O, false, true, V>::EB;
+            return AffShape<O, false, false, V>::EB;
+        };
+        return var == 1 ? shape(std::integral_constant<int, 1>{}) : shape(std::integral_constant<int, 0>{});
+    };
+    switch (order) {
+        case 2: return pick(std::integral_constant<int, 2>{});
+        case 3: return pick(std::integral_constant<int, 3>{});
+        case 4: return pick(std::integral_constant<int, 4>{});
+        default: return pick(std::integral_constant<int, 5>{});
+    }
+}
 
 // elements per block of an instantiation (block counts of the energy partials)
 template <typename R>
