@@ -1,4 +1,4 @@
-// The FP32 stage kernel of straight-sided meshes (TVD schemes).
+// The stage kernel of straight-sided meshes: FP32 TVD schemes and FP64.
 //
 // On a straight-sided tetrahedron the metric, the Jacobian and the face
 // scales are constant and the face frames orthonormal, so a stage's right-hand
@@ -16,10 +16,12 @@
 // moves that pattern, the same in every element, into the operators
 // (affine_mesh) and so keeps the reference's derivatives to rounding with one
 // metric per element.  Its face scales and frames vary by 2e-7 from single-
-// precision geometry; their mean changes seismograms by 3e-8 to 8e-8.  Meshes
-// that are not of this kind to 1e-6 are left to the general kernel.
+// precision geometry; their mean changes seismograms by 3e-8 to 8e-8, so FP32
+// takes the mean and the normal alone, FP64 every node's scale and the whole
+// frame.  Meshes that are not of this kind (affine_mesh) are left to the general
+// kernel.
 //
-// What bounds it: matrix and vector instructions share the SIMDs, and with
+// FP32, what bounds it: matrix and vector instructions share the SIMDs, and with
 // the general kernel the vector instructions were most of them (N = 3 elastic,
 // 64 shots: vector 44 %, matrix 25 % of the time, 1 TB/s).  So
 //   - the upwind flux is formed from the normal only (affine_flux): traction
@@ -47,6 +49,22 @@
 // large copy reaches 4.7).  Vector instructions are now 42 to 53 % of the time,
 // matrix instructions 15 to 29 %.  Order 1 stays with the general kernel (a
 // step of 4 values: no faster here).
+//
+// FP64: the same product on the FP64 matrix instruction, 64 cycles for 16 x 16 x
+// 4.  The general kernel spent a PML block's time (N = 4 with attenuation, stage
+// 2, 74k cycles) on loads and the PML update 31 %, face term 15 %, LIFT 7 %,
+// volume term and its metric 31 %, memory variables 13 %.  Here the face term runs
+// beside the PML update on the waves without nodes, and 15 columns in one product
+// replace 27 and the LIFT's 16 columns for 15 (9) values: 126 instead of 171 matrix
+// instructions a wave.  Where 16-row tiles and column tiles do not share out
+// evenly over four waves, the waves are split over the rows (row_groups: N = 5
+// a row tile each).  The flux is upwind_flux without divisions.
+// Per stage, before and after: N = 4 with attenuation and PML on 192,000 tets,
+// stages 1 and 2 1,975 -> 1,694 and 2,925 -> 2,553 us (2.3 and 2.5 TB/s; loads are
+// 38 % of a block's time, the product 25 %), N = 5 RK3 on 6,006 tets 176 -> 104
+// us in the PML and 56 -> 39 outside, N = 3 RK4 on 3,072 tets 16.5 -> 11.2 us, on 162
+// tets 11.3 -> 6.2 us (the last two also by smaller blocks, affine_shape_f64).
+// Three blocks per CU instead of two (168 registers): 1,762 and 2,877 us.
 #pragma once
 #include <type_traits>
 
@@ -157,22 +175,49 @@ constexpr unsigned long long kCofs[3] = {pack_nibbles(kCofX), pack_nibbles(kCofY
 
 // Block shape.  256 threads; node threads (element-in-block, node) hold the
 // fields, all four waves share the product.
-template <int ORDER, bool ATT, bool PML, int VAR>
+template <int ORDER, bool ATT, bool PML, typename R, int VAR>
 struct AffShape {
+    static constexpr bool F64 = sizeof(R) == 8;
     static constexpr int NP = Dims<ORDER>::NP, NPF = Dims<ORDER>::NPF, NFP = Dims<ORDER>::NFP;
     static constexpr int NTHR = 256, NW = 4;
     static constexpr int NCOL = ATT ? 15 : 9;       // columns of an element: rhs, memory-variable rates
     static constexpr int NV = NCOL;                 // odd: the node threads' row reads fall in different banks
     static constexpr int SFN = NFP | 1;             // face values: row of face nodes, odd
     static constexpr int ROWS = PML ? 9 + 27 : 9;   // q, and in the PML the contravariant fluxes [3][9]
-    static constexpr int BPC = VAR ? 2 : 4;         // blocks per CU the shape is sized for
+    // blocks per CU the shape is sized for; FP32: VAR 1 is the autotuner's
+    // alternative, FP64: VAR 1 and 2 have a half and a quarter of the elements
+    static constexpr int BPC = F64 || VAR ? 2 : 4;
     static constexpr int off_face(int eb) { return ROWS * eb * NP; }
     static constexpr int off_elem(int eb) {
         const int nt = eb * NP, f = off_face(eb) + eb * NCOL * SFN, v = nt * NV, e = 24 * nt + 4 * eb;
         return f > v ? (f > e ? f : e) : (v > e ? v : e);
     }
     static constexpr int lds_reals(int eb) { return off_elem(eb) + kAffElem * eb; }
+    // FP64: row tiles split over RG groups of waves, column tiles over the
+    // NW / RG waves of a group, for the fewest products of the busiest wave
+    static constexpr int RTV = (NP + 15) / 16;                      // row (node) tiles
+    static constexpr int products(int eb, int rg) {
+        const int ctl = (eb * NCOL + 15) / 16;
+        return ((RTV + rg - 1) / rg) * ((ctl + NW / rg - 1) / (NW / rg));
+    }
+    static constexpr int row_groups(int eb) {
+        int best = 1;
+        if (RTV >= 2 && products(eb, 2) < products(eb, best)) best = 2;
+        if (RTV >= 3 && products(eb, 4) < products(eb, best)) best = 4;
+        return best;
+    }
+    static constexpr int pick_f64() {
+        int eb = NTHR / NP;
+        if (PML && eb * NP > 192 && 192 / NP >= 2) eb = 192 / NP;
+        // a thread's face nodes in registers: two, in the PML five of the face waves
+        while (eb > 1 && (lds_reals(eb) * 8 + 8 * eb + 64 > 160 * 1024 / BPC ||
+                          eb * NFP > (PML ? 5 * 64 * (NW - (eb * NP + 63) / 64) : 2 * NTHR)))
+            --eb;
+        const int part = (eb + (1 << VAR) - 1) >> VAR;
+        return PML && part < 2 ? 2 : part;   // the last element's fluxes of two stages fit two elements' rows
+    }
     static constexpr int pick_eb() {
+        if (F64) return pick_f64();
         int eb = NTHR / NP;
         // Fewer elements where that fills the waves' column tiles better:
         // N = 4 with attenuation 4 elements in 4 tiles, one a wave (7 in 7
@@ -203,11 +248,12 @@ struct AffShape {
     static constexpr int LDS = lds_reals(EB);
     static constexpr int OFF_F = off_face(EB), OFF_E = off_elem(EB);
     static constexpr int NCT = EB * NCOL, CTL = (NCT + 15) / 16;   // columns, column tiles
-    static constexpr int RTV = (NP + 15) / 16;                      // row (node) tiles
     // values of a lane: 3 per node 4 ks + l/16, then one per face node; in steps of 8
     static constexpr int KS = (NP + 3) / 4, KSV = 3 * KS, KSL = NFP / 4, KT = KSV + KSL, NS = (KT + 7) / 8;
     static constexpr int CPW = (CTL + NW - 1) / NW;    // column tiles of a wave
     static constexpr int TG = RTV > 2 ? 1 : 2;   // column tiles in one pass (accumulator registers)
+    static constexpr int RG = F64 ? row_groups(EB) : 1, RW = (RTV + RG - 1) / RG;   // row tiles of a wave
+    static constexpr int CG = NW / RG, CW = (CTL + CG - 1) / CG;                    // FP64: its column tiles
 };
 
 
@@ -221,21 +267,22 @@ __device__ __forceinline__ void block_barrier() {
 // RC: the recomputing RK2 kernels (stage_kernel in plain_kernels.hpp says
 // what they leave out; here without attenuation or PML they only fix the
 // stage), 0: any stage of any TVD scheme.
-template <int ORDER, bool ATT, bool PML, int VAR, int RC>
-__global__ void __launch_bounds__(256, (AffShape<ORDER, ATT, PML, VAR>::BPC))
-affine_kernel(StageArgs<float> a) {
-    using S = AffShape<ORDER, ATT, PML, VAR>;
+template <int ORDER, bool ATT, bool PML, typename R, bool LS, int VAR, int RC>
+__global__ void __launch_bounds__(256, (AffShape<ORDER, ATT, PML, R, VAR>::BPC))
+affine_kernel(StageArgs<R> a) {
+    using S = AffShape<ORDER, ATT, PML, R, VAR>;
+    constexpr bool F64 = S::F64, WEIGHTED = !F64;
     constexpr int NP = S::NP, NPF = S::NPF, NFP = S::NFP, EB = S::EB, NT = S::NT, SFN = S::SFN, NCOL = S::NCOL, NV = S::NV;
     constexpr int NTHR = S::NTHR, NW = S::NW, FIT = S::FIT, NFT = S::NFT, NFN = S::NFN;
     // planes through buffer descriptors with PML or attenuation; without, the
     // few loads of a thread come out 2 % faster as global ones
     constexpr bool BUF = PML || ATT;
-    __shared__ __align__(16) float lds[S::LDS];
-    float *sQ = lds;                        // [9][NT]
-    float *sC = lds + 9 * NT;               // [3][9][NT] contravariant fluxes (PML)
-    float *sF = lds + S::OFF_F;             // [EB][NCOL][SFN] face values
-    float *sE = lds + S::OFF_E;             // [EB][kAffElem]
-    float *sV = lds;                        // [NT][NV] the product, over everything before sE
+    __shared__ __align__(16) R lds[S::LDS];
+    R *sQ = lds;                        // [9][NT]
+    R *sC = lds + 9 * NT;               // [3][9][NT] contravariant fluxes (PML)
+    R *sF = lds + S::OFF_F;             // [EB][NCOL][SFN] face values
+    R *sE = lds + S::OFF_E;             // [EB][kAffElem]
+    R *sV = lds;                        // [NT][NV] the product, over everything before sE
     static_assert(24 * NT + 4 * EB <= S::OFF_E, "energy values must fit the LDS");
 
     const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -246,11 +293,11 @@ affine_kernel(StageArgs<float> a) {
     const unsigned per = nb / kXcds, extra = nb % kXcds;
     const unsigned lb = xcd * per + (xcd < extra ? xcd : extra) + rank;
     const int shot = (int)(lb % (unsigned)a.nshot), eblk = (int)(lb / (unsigned)a.nshot);
-    const float *qin = a.qin + (size_t)shot * 9 * ng;
-    const float *qbase = a.qbase + (size_t)shot * 9 * ng;
-    float *qout = a.qout + (size_t)shot * 9 * ng;
-    const float *matc = a.matc + (size_t)shot * a.mat_stride;
-    const unsigned pnb = (unsigned)(ng * sizeof(float));
+    const R *qin = a.qin + (size_t)shot * 9 * ng;
+    const R *qbase = a.qbase + (size_t)shot * 9 * ng;
+    R *qout = a.qout + (size_t)shot * 9 * ng;
+    const R *matc = a.matc + (size_t)shot * a.mat_stride;
+    const unsigned pnb = (unsigned)(ng * sizeof(R));
     const unsigned pnb_base = RC == 1 || (RC == 0 && a.irk == 1) ? 0u : pnb;
 
     const bool node_thr = t < NT;
@@ -260,32 +307,33 @@ affine_kernel(StageArgs<float> a) {
     const int e = valid ? a.elist[idx] : 0;
     const unsigned g32 = (unsigned)e * NP + j;
     const size_t g = (size_t)e * NP + j;
-    const float dt = a.dt_elem ? a.dt_elem[e] : a.dt;
+    const R dt = a.dt_elem ? a.dt_elem[e] : a.dt;
 
     // Element constants into LDS.  Elements past the end of the list take
     // element 0's; their values are finite and never stored.
     auto stage_elements = [&](int th, int nth) {
         for (int i = th; i < EB; i += nth) {
             const int b = eblk * EB + i, ee = b < a.nlist ? a.elist[b] : 0;
-            const float *m = a.emet + (size_t)ee * 12, *mc = matc + (size_t)ee * 8;
-            float met[9];
+            const R *m = a.emet + (size_t)ee * 12, *mc = matc + (size_t)ee * 8;
+            R met[9];
 #pragma unroll
             for (int k = 0; k < 9; ++k) met[k] = m[k];
-            const float vp = mc[0], vs = mc[1], lam = mc[3], mu = mc[4], lvl = mc[5], irho = mc[6];
-            float *el = sE + i * kAffElem;
+            const R vp = mc[0], vs = mc[1], lam = mc[3], mu = mc[4], lvl = mc[5], irho = mc[6];
+            R *el = sE + i * kAffElem;
 #pragma unroll
             for (int k = 0; k < 9; ++k) el[AE_MET + k] = met[k];
-            el[AE_COEF + 0] = -(lam + 2.f * mu); el[AE_COEF + 1] = -lam; el[AE_COEF + 2] = -mu; el[AE_COEF + 3] = -irho;
-            el[AE_COEF + 4] = 0.f; el[AE_COEF + 5] = -1.f; el[AE_COEF + 6] = -0.5f;
+            el[AE_COEF + 0] = -(lam + R(2) * mu); el[AE_COEF + 1] = -lam; el[AE_COEF + 2] = -mu; el[AE_COEF + 3] = -irho;
+            el[AE_COEF + 4] = R(0); el[AE_COEF + 5] = -R(1); el[AE_COEF + 6] = -R(0.5);
             el[AE_VP] = vp; el[AE_VS] = vs; el[AE_LAM] = lam; el[AE_MU] = mu; el[AE_LVL] = lvl;
-            if constexpr (ATT) { el[AE_P1] = irho / vp; el[AE_P2] = 0.5f * irho / vs; }
+            if constexpr (ATT) { el[AE_P1] = irho / vp; el[AE_P2] = R(0.5) * irho / vs; }
         }
     };
 
     // The face nodes of thread th of the face term: what does not depend on
     // this block's own values, the neighbour traces among it
-    float fq[FIT][9];
-    f32x4_t fg[FIT];
+    R fq[FIT][9];
+    f32x4_t fg[F64 ? 1 : FIT];
+    R ffr[F64 ? FIT : 1][9], ffs[F64 ? FIT : 1];
     int fnb[FIT], fown[FIT];
     auto face_load = [&](int th) {
         int fe[FIT];
@@ -298,13 +346,19 @@ affine_kernel(StageArgs<float> a) {
         for (int i = 0; i < FIT; ++i) {
             const int q = th + NFT * i, qq = q < NFN ? q : 0, fb = qq / NFP, k = qq - fb * NFP;
             fnb[i] = a.nbrt[(size_t)fe[i] * NFP + k];
-            fg[i] = *reinterpret_cast<const f32x4_t *>(a.fgeo + ((size_t)fe[i] * 4 + k / NPF) * 4);
+            if constexpr (F64) {
+                ffs[i] = a.fscale[(size_t)fe[i] * NFP + k];
+#pragma unroll
+                for (int c = 0; c < 9; ++c) ffr[i][c] = a.frame[((size_t)fe[i] * 4 + k / NPF) * 9 + c];
+            } else {
+                fg[i] = *reinterpret_cast<const f32x4_t *>(a.fgeo + ((size_t)fe[i] * 4 + k / NPF) * 4);
+            }
             fown[i] = fb * NP + a.fmask[k];
         }
 #pragma unroll
         for (int i = 0; i < FIT; ++i) {
             // a boundary face's index is past every plane: its loads return 0
-            const unsigned gn = fnb[i] >= 0 ? (unsigned)fnb[i] : 0x3fffffffu;
+            const unsigned gn = fnb[i] >= 0 ? (unsigned)fnb[i] : 0xffffffffu / (unsigned)sizeof(R);
 #pragma unroll
             for (int f = 0; f < 9; ++f) fq[i][f] = pload<true>(qin + f * ng, pnb, gn);
         }
@@ -316,24 +370,30 @@ affine_kernel(StageArgs<float> a) {
             if (q < NFN) {
                 const int fb = q / NFP, k = q - fb * NFP;
                 const bool fvalid = eblk * EB + fb < a.nlist;
-                float dq[9], fl[NCOL];
+                R dq[9], fl[NCOL];
 #pragma unroll
                 for (int f = 0; f < 9; ++f) {
                     dq[f] = fq[i][f] - sQ[f * NT + fown[i]];
                 }
-                const float *el = sE + fb * kAffElem;
+                const R *el = sE + fb * kAffElem;
                 // the jump of a boundary face is its own trace, here with the
                 // other sign; absorbing faces (-2) change the sign once more
-                const float fs = fvalid ? (fnb[i] == -1 ? -fg[i][3] : fg[i][3]) : 0.f;
-                affine_flux<ATT>(fg[i][0], fg[i][1], fg[i][2], fs, el, el[AE_COEF + 3], fnb[i] == -1, dq, fl);
-                float *dst = sF + fb * NCOL * SFN + k;
+                if constexpr (F64) {
+                    const R fs = fvalid ? (fnb[i] == -1 ? R(-0.5) : R(0.5)) * ffs[i] : R(0);
+                    upwind_flux<R>(ffr[i], el[AE_VP], el[AE_VS], el[AE_LAM], el[AE_MU], el[AE_LVL], -el[AE_COEF + 3],
+                                   el[AE_P1], el[AE_P2], fnb[i] == -1, fs, dq, fl, fl + (ATT ? 9 : 0), ATT);
+                } else {
+                    const R fs = fvalid ? (fnb[i] == -1 ? -fg[i][3] : fg[i][3]) : R(0);
+                    affine_flux<ATT>(fg[i][0], fg[i][1], fg[i][2], fs, el, el[AE_COEF + 3], fnb[i] == -1, dq, fl);
+                }
+                R *dst = sF + fb * NCOL * SFN + k;
 #pragma unroll
                 for (int f = 0; f < NCOL; ++f) dst[f * SFN] = fl[f];
             }
         }
     };
 
-    float qs[9];
+    R qs[9];
     int src_first = -1, rec_slot_e = -1;
     auto node_load = [&]() {
         src_first = a.src_head[(size_t)shot * (a.nglob / NP) + e];
@@ -370,12 +430,12 @@ affine_kernel(StageArgs<float> a) {
             constexpr bool LASTF = RC != 1;
             constexpr int NLASTF = RC == 2 ? 54 * NP : 27 * NP, NLS = LASTF ? (NLASTF + NNT - 1) / NNT : 1;
             static_assert(!LASTF || NLASTF <= 27 * NT, "last-element fluxes must fit the flux rows");
-            float *sLast = sC, *sLast1 = sC + 27 * NP;
-            float lst[NLS];
+            R *sLast = sC, *sLast1 = sC + 27 * NP;
+            R lst[NLS];
             if constexpr (LASTF) {
                 if (a.pml_compat) {
-                    const float *lf = a.last_flux + (size_t)shot * 27 * NP;
-                    const float *lf1 = RC == 2 ? a.last_flux1 + (size_t)shot * 27 * NP : lf;
+                    const R *lf = a.last_flux + (size_t)shot * 27 * NP;
+                    const R *lf1 = RC == 2 ? a.last_flux1 + (size_t)shot * 27 * NP : lf;
 #pragma unroll
                     for (int r = 0; r < NLS; ++r) {
                         const int i = t + r * NNT;
@@ -384,13 +444,13 @@ affine_kernel(StageArgs<float> a) {
                     }
                 }
             }
-            const float *pin = a.pin + (size_t)shot * 27 * ng;
-            const float *pbase = a.pbase + (size_t)shot * 27 * ng;
-            float *pout = a.pout + (size_t)shot * 27 * ng;
-            float pc[9], cur[27], bse[RC == 0 ? 27 : 1], mv[9], lam = 0, mu = 0, irho = 0;
+            const R *pin = a.pin + (size_t)shot * 27 * ng;
+            const R *pbase = a.pbase + (size_t)shot * 27 * ng;
+            R *pout = a.pout + (size_t)shot * 27 * ng;
+            R pc[9], cur[27], bse[RC == 0 ? 27 : 1], mv[9], lam = 0, mu = 0, irho = 0;
             if (node_thr) {
                 node_load();
-                const float *pmlc = a.pmlc + (size_t)shot * a.pmlc_stride_ng * ng;
+                const R *pmlc = a.pmlc + (size_t)shot * a.pmlc_stride_ng * ng;
 #pragma unroll
                 for (int k = 0; k < 9; ++k) pc[k] = pload<BUF>(pmlc + k * ng, pnb, g32);
 #pragma unroll
@@ -399,8 +459,9 @@ affine_kernel(StageArgs<float> a) {
 #pragma unroll
                     for (int c = 0; c < 27; ++c) bse[c] = pload<BUF>(pbase + c * ng, pnb_base, g32);
                 }
-                const f32x4_t *m4 = reinterpret_cast<const f32x4_t *>(a.emet + (size_t)e * 12);
-                const f32x4_t ma = m4[0], mb = m4[1], mc = m4[2];
+                typedef R r4 __attribute__((ext_vector_type(4)));
+                const r4 *m4 = reinterpret_cast<const r4 *>(a.emet + (size_t)e * 12);
+                const r4 ma = m4[0], mb = m4[1], mc = m4[2];
 #pragma unroll
                 for (int k = 0; k < 4; ++k) { mv[k] = ma[k]; mv[4 + k] = mb[k]; }
                 mv[8] = mc[0];
@@ -416,47 +477,54 @@ affine_kernel(StageArgs<float> a) {
             }
             if (node_thr) node_store();
             block_barrier();
-            float cf[27];
+            R cf[27];
             if (node_thr) {
                 // modified fluxes and the ADE update of f',g',h', as in
                 // stage_kernel (src/timeloopMod.f90:399-405, src/rungekuttaMod.f90:52-63)
-                float Fm[9], Gm[9], Hm[9];
-                elastic_flux_node(qs, -(lam + 2.f * mu), -lam, -mu, -irho, Fm, Gm, Hm);
-                const RkStage<float> rs = rk_stage<float, RC>(a.scheme, a.irk, a.w13, a.w23, 0.f, 0.f);
+                R Fm[9], Gm[9], Hm[9];
+                elastic_flux_node(qs, -(lam + R(2) * mu), -lam, -mu, -irho, Fm, Gm, Hm);
+                const RkStage<R> rs = rk_stage<R, RC>(a.scheme, a.irk, a.w13, a.w23, a.lsa, a.lsb);
                 const bool on = !a.pml_on || a.pml_on[shot] != 0;
 #pragma unroll
                 for (int d = 0; d < 3; ++d) {
-                    float pv[9];
-                    const float al = on ? pc[d] : 0.f, dk = on ? pc[3 + d] : 0.f;
-                    const float rk = on ? 1.f / pc[6 + d] : 1.f;
-                    const float *FF = d == 0 ? Fm : (d == 1 ? Gm : Hm);
+                    R pv[9];
+                    const R al = on ? pc[d] : R(0), dk = on ? pc[3 + d] : R(0);
+                    const R rk = on ? R(1) / pc[6 + d] : R(1);
+                    const R *FF = d == 0 ? Fm : (d == 1 ? Gm : Hm);
                     const int skip = d == 0 ? 4 : (d == 1 ? 5 : 3);   // identically zero
 #pragma unroll
                     for (int i = 0; i < 9; ++i) {
                         const int c = d * 9 + i;
-                        float c0 = on ? cur[c] : 0.f;
+                        R c0 = on ? cur[c] : R(0);
                         if constexpr (RC == 2) {
-                            const float dadt1 = -al * c0 - dk * (c0 + sLast1[c * NP + j]);
-                            float none = 0;
-                            c0 = rk_update<float, false, false, 1>(rs, c0, none, dadt1, dt);
+                            const R dadt1 = -al * c0 - dk * (c0 + sLast1[c * NP + j]);
+                            R none = 0;
+                            c0 = rk_update<R, false, false, 1>(rs, c0, none, dadt1, dt);
                         }
-                        const float mod = (c0 + FF[i]) * rk;
+                        const R mod = (c0 + FF[i]) * rk;
 #pragma unroll
                         for (int o = 0; o < 3; ++o) {
-                            const float m = mv[3 * o + d];
-                            if (d == 0) cf[o * 9 + i] = i != skip ? m * mod : 0.f;
+                            const R m = mv[3 * o + d];
+                            if (d == 0) cf[o * 9 + i] = i != skip ? m * mod : R(0);
                             else if (i != skip) cf[o * 9 + i] = cf[o * 9 + i] + m * mod;
                         }
                         if constexpr (RC == 1) continue;
-                        const float lastv = sLast[c * NP + j];
-                        const float u = RC == 2 || a.pml_compat ? lastv : mod;
-                        const float dadt = -al * c0 - dk * (c0 + u);
-                        if constexpr (RC == 2) pv[i] = rk_update<float, false, false, 2>(rs, c0, cur[c], dadt, dt);
-                        else if constexpr (RC == 0) pv[i] = rk_update<float, false>(rs, c0, bse[c], dadt, dt);
+                        const R lastv = sLast[c * NP + j];
+                        const R u = RC == 2 || a.pml_compat ? lastv : mod;
+                        const R dadt = -al * c0 - dk * (c0 + u);
+                        if constexpr (RC == 2) pv[i] = rk_update<R, false, false, 2>(rs, c0, cur[c], dadt, dt);
+                        else if constexpr (RC == 0) pv[i] = rk_update<R, LS>(rs, c0, bse[c], dadt, dt);
                     }
                     if (RC != 1 && valid) {
 #pragma unroll
                         for (int i = 0; i < 9; ++i) pstore<BUF>(pout + (d * 9 + i) * ng, pnb, g32, pv[i]);
+                    }
+                    if constexpr (LS) {
+                        if (valid) {
+                            R *pres = a.pres + (size_t)shot * 27 * ng;
+#pragma unroll
+                            for (int i = 0; i < 9; ++i) pstore<BUF>(pres + (d * 9 + i) * ng, pnb, g32, bse[d * 9 + i]);
+                        }
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 }
@@ -474,10 +542,93 @@ affine_kernel(StageArgs<float> a) {
     }
 
     // ---- the product -----------------------------------------------------
+    constexpr int RTV = S::RTV, CTL = S::CTL;
+    if constexpr (F64) {
+        // Wave w takes row tiles RW (w % RG).. and column tiles w / RG, w / RG +
+        // CG, ..: at value s of its column's list a lane supplies one B value,
+        // and the operator's fragments of the wave's row tiles load PREF values
+        // ahead.
+        constexpr int RW = S::RW, RG = S::RG, CW = S::CW, CG = S::CG, KT = S::KT, PREF = 12 / RW;
+        typedef double f64x4_t __attribute__((ext_vector_type(4)));
+        const int r0 = (w % RG) * RW, c0 = w / RG;
+        const double *ak = reinterpret_cast<const double *>(a.AK) + lane;
+        double af[PREF][RW];
+        auto load_a = [&](int s) {
+#pragma unroll
+            for (int r = 0; r < RW; ++r) af[s % PREF][r] = ak[(s * RTV + (r0 + r < RTV ? r0 + r : RTV - 1)) * 64];
+        };
+#pragma unroll
+        for (int s = 0; s < PREF; ++s) load_a(s);
+        __syncthreads();   // q, flux rows and face values are in LDS
+        f64x4_t acc[CW][RW];
+        R K[CW][9], C[CW][3];
+        int row[CW][3], lrow[CW];
+#pragma unroll
+        for (int c = 0; c < CW; ++c) {
+            const int col = (c0 + c * CG) * 16 + (lane & 15);
+            const bool cok = col < S::NCT;
+            const int ce = cok ? col / NCOL : 0, cc = cok ? col - (col / NCOL) * NCOL : 0;
+            lrow[c] = S::OFF_F + (ce * NCOL + cc) * SFN + (lane >> 4);
+            const R *el = sE + ce * kAffElem;
+            const bool flux = PML && cc < 9;   // stored contravariant fluxes
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const R cof = el[AE_COEF + (int)((kCofs[k] >> (4 * cc)) & 15)];
+                row[c][k] = (flux ? (9 + 9 * k + cc) : (int)((kRows[k] >> (4 * cc)) & 15)) * NT + ce * NP;
+#pragma unroll
+                for (int o = 0; o < 3; ++o) {
+                    const R m = el[AE_MET + 3 * o + k] * cof;
+                    K[c][3 * o + k] = flux ? (o == k ? R(1) : R(0)) : m;
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < RW; ++r) acc[c][r] = f64x4_t{0, 0, 0, 0};
+        }
+#pragma unroll
+        for (int s = 0; s < KT; ++s) {
+#pragma unroll
+            for (int c = 0; c < CW; ++c) {
+                R v;
+                if (s < S::KSV) {
+                    if (s % 3 == 0) {
+                        const int m = 4 * (s / 3) + (lane >> 4);
+                        const int mm = 4 * (s / 3) + 3 < NP || m < NP ? m : 0;   // the operator is zero beyond Np
+                        const R x = lds[row[c][0] + mm], y = lds[row[c][1] + mm], z = lds[row[c][2] + mm];
+#pragma unroll
+                        for (int o = 0; o < 3; ++o)
+                            C[c][o] = K[c][3 * o] * x + K[c][3 * o + 1] * y + K[c][3 * o + 2] * z;
+                    }
+                    v = C[c][s % 3];
+                } else {
+                    v = lds[lrow[c] + 4 * (s - S::KSV)];
+                }
+#pragma unroll
+                for (int r = 0; r < RW; ++r) acc[c][r] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[s % PREF][r], v, acc[c][r], 0, 0, 0);
+            }
+            if (s + PREF < KT) load_a(s + PREF);
+            if (s % 3 == 2) __builtin_amdgcn_sched_barrier(0);
+        }
+        __syncthreads();   // everything before the element constants is dead
+        // accumulator element v: node row 4v + l/16 of the row tile, column l%16
+#pragma unroll
+        for (int c = 0; c < CW; ++c) {
+            const int col = (c0 + c * CG) * 16 + (lane & 15);
+            if (col < S::NCT) {
+                const int ce = col / NCOL, cc = col - ce * NCOL;
+#pragma unroll
+                for (int r = 0; r < RW; ++r)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        const int node = (r0 + r) * 16 + 4 * v + (lane >> 4);
+                        if (node < NP) sV[(ce * NP + node) * NV + cc] = acc[c][r][v];
+                    }
+            }
+        }
+    } else {
     // Each wave takes column tiles w, w+4, .. against all row tiles, TG of
     // them at a time.  Unit u = (step u / RTV, row tile u % RTV): its three
     // A parts load PREF units ahead.
-    constexpr int RTV = S::RTV, CPW = S::CPW, CTL = S::CTL, NU = S::NS * RTV, PREF = 2;
+    constexpr int CPW = S::CPW, NU = S::NS * RTV, PREF = 2;
     const u32x4_t *ak = reinterpret_cast<const u32x4_t *>(a.AK) + lane;
     bf16x8_t af[PREF + 1][3];
     auto load_a = [&](int u) {
@@ -600,16 +751,17 @@ affine_kernel(StageArgs<float> a) {
                 }
         }
     }
+    }
 
     // ---- node threads: memory variables, sources, Runge-Kutta update -------
-    float th[ATT ? 18 : 1], thb[ATT && RC == 0 ? 18 : 1], gi[ATT && RC == 2 ? 6 : 1], avc[ATT ? 9 : 1];
-    float qb[9], alo[9], blo[9];
+    R th[ATT ? 18 : 1], thb[ATT && RC == 0 ? 18 : 1], gi[ATT && RC == 2 ? 6 : 1], avc[ATT ? 9 : 1];
+    R qb[9], alo[9], blo[9];
     const bool comp = a.qlo_out != nullptr;
     const unsigned nel = (unsigned)(ng / NP);
     if (node_thr) {
         if constexpr (ATT) {
-            const float *thin = a.thin + (size_t)shot * 18 * ng;
-            const float *av = a.anel + (size_t)shot * a.anel_stride;
+            const R *thin = a.thin + (size_t)shot * 18 * ng;
+            const R *av = a.anel + (size_t)shot * a.anel_stride;
 #pragma unroll
             for (int c = 0; c < 18; ++c) th[c] = pload<BUF>(thin + c * ng, pnb, g32);
             if constexpr (RC == 2) {
@@ -621,7 +773,7 @@ affine_kernel(StageArgs<float> a) {
                 for (int c = 0; c < 18; ++c) thb[c] = pload<BUF>(a.thbase + ((size_t)shot * 18 + c) * ng, pnb_base, g32);
             }
 #pragma unroll
-            for (int c = 0; c < 9; ++c) avc[c] = pload<BUF>(av, nel * (unsigned)(NMB * 3 * sizeof(float)), (unsigned)e * (NMB * 3) + c);
+            for (int c = 0; c < 9; ++c) avc[c] = pload<BUF>(av, nel * (unsigned)(NMB * 3 * sizeof(R)), (unsigned)e * (NMB * 3) + c);
         }
         if constexpr (RC != 1) {
 #pragma unroll
@@ -637,28 +789,28 @@ affine_kernel(StageArgs<float> a) {
         }
     }
     __syncthreads();
-    float qnew[9], rhs[9];
+    R qnew[9], rhs[9];
     if (node_thr) {
-        const float *v = sV + t * NV;
+        const R *v = sV + t * NV;
 #pragma unroll
         for (int i = 0; i < 9; ++i) rhs[i] = v[i];
-        const RkStage<float> rs = rk_stage<float, RC>(a.scheme, a.irk, a.w13, a.w23, 0.f, 0.f);
+        const RkStage<R> rs = rk_stage<R, RC>(a.scheme, a.irk, a.w13, a.w23, a.lsa, a.lsb);
         if constexpr (ATT) {
-            float gn[6];
+            R gn[6];
 #pragma unroll
             for (int c = 0; c < 6; ++c) gn[c] = v[9 + c];
             // one mechanism at a time (src/timeloopMod.f90:426-461): every
             // memory variable advances by w (g - theta)
 #pragma unroll
             for (int i = 0; i < NMB; ++i) {
-                const float wl = a.wl[i], a1 = avc[i * 3 + 0], a2 = avc[i * 3 + 1], a3 = avc[i * 3 + 2];
-                float tm[6];
+                const R wl = a.wl[i], a1 = avc[i * 3 + 0], a2 = avc[i * 3 + 1], a3 = avc[i * 3 + 2];
+                R tm[6];
 #pragma unroll
                 for (int c = 0; c < 6; ++c) {
                     tm[c] = th[i * 6 + c];
                     if constexpr (RC == 2) {
-                        float none = 0;
-                        tm[c] = rk_update<float, false, false, 1>(rs, tm[c], none, wl * (gi[c] - tm[c]), dt);
+                        R none = 0;
+                        tm[c] = rk_update<R, false, false, 1>(rs, tm[c], none, wl * (gi[c] - tm[c]), dt);
                     }
                 }
                 rhs[0] = rhs[0] + a3 * tm[0] + a1 * (tm[1] + tm[2]);
@@ -671,9 +823,9 @@ affine_kernel(StageArgs<float> a) {
 #pragma unroll
                     for (int c = 0; c < 6; ++c) {
                         const int k = i * 6 + c;
-                        const float r = wl * (gn[c] - tm[c]);
-                        if constexpr (RC == 2) th[k] = rk_update<float, false, true, 2>(rs, tm[c], th[k], r, dt);
-                        else th[k] = rk_update<float, false, true>(rs, tm[c], thb[k], r, dt);
+                        const R r = wl * (gn[c] - tm[c]);
+                        if constexpr (RC == 2) th[k] = rk_update<R, false, WEIGHTED, 2>(rs, tm[c], th[k], r, dt);
+                        else th[k] = rk_update<R, LS, WEIGHTED>(rs, tm[c], thb[k], r, dt);
                     }
                 }
             }
@@ -685,16 +837,20 @@ affine_kernel(StageArgs<float> a) {
 #pragma unroll
                     for (int k = 0; k < 18; ++k) pstore<BUF>(a.thout + ((size_t)shot * 18 + k) * ng, pnb, g32, th[k]);
                 }
+                if constexpr (LS) {
+#pragma unroll
+                    for (int k = 0; k < 18; ++k) pstore<BUF>(a.thres + ((size_t)shot * 18 + k) * ng, pnb, g32, thb[k]);
+                }
             }
         }
         if (valid) add_sources<NP>(a, shot, j, src_first, it_step, rhs);
-        if (comp) {
+        if (!LS && comp) {
             const int scheme = RC ? 2 : a.scheme, irk = RC ? RC : a.irk;
 #pragma unroll
             for (int f = 0; f < 9; ++f) {
-                float lo;
-                const float b = RC == 1 ? qs[f] : qb[f], bl = RC == 1 ? alo[f] : blo[f];
-                rk_combine_comp<float>(scheme, irk, qs[f], alo[f], b, bl, rhs[f], dt, a.w13, a.w23, qnew[f], lo);
+                R lo;
+                const R b = RC == 1 ? qs[f] : qb[f], bl = RC == 1 ? alo[f] : blo[f];
+                rk_combine_comp<R>(scheme, irk, qs[f], alo[f], b, bl, rhs[f], dt, a.w13, a.w23, qnew[f], lo);
                 if (valid) {
                     pstore<BUF>(qout + f * ng, pnb, g32, qnew[f]);
                     pstore<BUF>(a.qlo_out + ((size_t)shot * 9 + f) * ng, pnb, g32, lo);
@@ -703,12 +859,16 @@ affine_kernel(StageArgs<float> a) {
         } else {
 #pragma unroll
             for (int f = 0; f < 9; ++f) {
-                if constexpr (RC == 1) qb[f] = 0.f;
-                qnew[f] = rk_update<float, false, true, RC>(rs, qs[f], qb[f], rhs[f], dt);
+                if constexpr (RC == 1) qb[f] = R(0);
+                qnew[f] = rk_update<R, LS, WEIGHTED, RC>(rs, qs[f], qb[f], rhs[f], dt);
             }
             if (valid) {
 #pragma unroll
                 for (int f = 0; f < 9; ++f) pstore<BUF>(qout + f * ng, pnb, g32, qnew[f]);
+                if constexpr (LS) {
+#pragma unroll
+                    for (int f = 0; f < 9; ++f) pstore<BUF>(a.qres + ((size_t)shot * 9 + f) * ng, pnb, g32, qb[f]);
+                }
             }
         }
     }
@@ -724,7 +884,7 @@ affine_kernel(StageArgs<float> a) {
             if (rec_slot_e >= 0) update_receiver<NP>(a, shot, j, rec_slot_e, dt, qnew, rhs);
         }
         if (a.blk_energy) {
-            const float rho = node_thr ? matc[(size_t)e * 8 + 2] : 1.f;
+            const R rho = node_thr ? matc[(size_t)e * 8 + 2] : R(1);
             block_energy<ORDER, EB, NTHR>(a, lds, shot, eblk, node_thr, valid, t, eb, j, e, rho, qnew);
         }
     }

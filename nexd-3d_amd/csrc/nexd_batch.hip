@@ -54,7 +54,8 @@ struct Batch : BatchBase {
     R *paux[2] = {nullptr, nullptr};
     R *D = nullptr, *DK = nullptr, *LT = nullptr, *mass = nullptr, *metric = nullptr, *fscale = nullptr, *frame = nullptr;
     R *jac = nullptr;
-    unsigned short *AK = nullptr;                        // affine kernels (straight-sided meshes, FP32)
+    unsigned short *AK = nullptr;                        // affine kernels (straight-sided meshes): FP32, FP64 operators
+    double *AD = nullptr;
     R *emet = nullptr, *fgeo = nullptr;
     int *nbrt = nullptr;
     bool affine = false;
@@ -198,7 +199,9 @@ struct Batch : BatchBase {
     // element blocks of one list launch (per shot)
     int nblocks(int n, bool pml) const {
         if (affine) {
-            const int eb = nexd::affine_eb(cfg.order, cfg.attenuation != 0, pml, tile);
+            const bool att = cfg.attenuation != 0;
+            const int var = sizeof(R) == 8 ? nexd::affine_shape_f64(cfg.order, att, pml, (long)n * cfg.nshot) : tile;
+            const int eb = nexd::affine_block<R>(cfg.order, att, pml, var).eb;
             return (n + eb - 1) / eb;
         }
         return nexd::stage_blocks<R>(cfg.order, n, cfg.attenuation != 0, pml, tile);
@@ -220,8 +223,9 @@ struct Batch : BatchBase {
 
     // the affine kernels' operators, from the uploaded ones and the mesh
     int put_affine_operators() {
-        return upload(&AK, nexd::mfma_affine_fragments(nexd::affine_operators(ops_host.D, np, affine_comb), ops_host.LT, np,
-                                                       4 * npf));
+        const std::vector<double> d = nexd::affine_operators(ops_host.D, np, affine_comb);
+        if (sizeof(R) == 8) return upload(&AD, nexd::mfma_affine_fragments_f64(d, ops_host.LT, np, 4 * npf));
+        return upload(&AK, nexd::mfma_affine_fragments(d, ops_host.LT, np, 4 * npf));
     }
 
     void count_blocks() { nblk_total = nblocks(n_plain, false) + nblocks(n_pml, true); }
@@ -282,19 +286,22 @@ struct Batch : BatchBase {
         a.mass = mass; a.jac = jac; a.emat = emat;
         a.emat_stride = cfg.shared_material ? 0 : cfg.nelem * 2;
         a.pml_on = cfg.pml ? pml_on : nullptr;
-        a.AK = AK; a.emet = emet; a.fgeo = fgeo; a.nbrt = nbrt;
+        a.AK = sizeof(R) == 8 ? (const void *)AD : (const void *)AK; a.emet = emet; a.fgeo = fgeo; a.nbrt = nbrt;
         return a;
     }
 
     void dispatch(const nexd::StageArgs<R> &a, bool pml) { dispatch(a, pml, stream); }
     void dispatch(const nexd::StageArgs<R> &a, bool pml, hipStream_t s) {
         const bool att = cfg.attenuation != 0;
-        if constexpr (sizeof(R) == 4) {
-            if (affine) {
-                if (tile == 1) nexd::launch_affine<1>(cfg.order, att, pml, a, s);
-                else nexd::launch_affine<0>(cfg.order, att, pml, a, s);
-                return;
+        if (affine) {
+            if constexpr (sizeof(R) == 8) {
+                nexd::launch_affine_f64(cfg.order, att, pml, a, s);
+            } else if (tile == 1) {
+                nexd::launch_affine<float, false, 1>(cfg.order, att, pml, a, s);
+            } else {
+                nexd::launch_affine<float, false, 0>(cfg.order, att, pml, a, s);
             }
+            return;
         }
         if (a.scheme == NEXD_LSRK4) {
             nexd::launch_stage<R, true, 0>(cfg.order, att, pml, a, s);
@@ -674,16 +681,18 @@ int upload_mesh(Batch<R> *b, const int *ibool, const double *const met[9], const
     if (!err.empty())
         return err[0] == '!' ? b->fail(NEXD_E_UNSUPPORTED, err.substr(1)) : b->fail(NEXD_E_ARG, err);
     int rc;
-    // straight-sided meshes take the affine kernels in FP32 (TVD schemes, order
-    // 2 and up), every other the general ones
+    // straight-sided meshes take the affine kernels (order 2 and up; FP32: TVD
+    // schemes), every other the general ones
     nexd::AffineHost ah;
-    const bool affine = sizeof(R) == 4 && b->cfg.timeint != NEXD_LSRK4 && b->cfg.order >= nexd::kAffMinOrder &&
-                        nexd::affine_mesh(m, b->cfg.nelem, b->np, b->npf, ah);
+    constexpr bool f64 = sizeof(R) == 8;
+    const bool affine = (f64 || b->cfg.timeint != NEXD_LSRK4) && b->cfg.order >= nexd::kAffMinOrder &&
+                        nexd::affine_mesh(m, b->cfg.nelem, b->np, b->npf, f64, ah);
     if ((rc = b->upload(&b->jac, cvt<R>(m.jac)))) return rc;
     if (affine) {
         b->affine_comb = ah.comb;
         if ((rc = b->put_affine_operators()) || (rc = b->upload(&b->emet, cvt<R>(ah.emet))) ||
-            (rc = b->upload(&b->fgeo, cvt<R>(ah.fgeo))) || (rc = b->upload(&b->nbrt, ah.nbrt)))
+            (!f64 && (rc = b->upload(&b->fgeo, cvt<R>(ah.fgeo)))) || (rc = b->upload(&b->nbrt, ah.nbrt)) ||
+            (f64 && ((rc = b->upload(&b->fscale, cvt<R>(m.fscale))) || (rc = b->upload(&b->frame, cvt<R>(m.frame))))))
             return rc;
     } else if ((rc = b->upload(&b->metric, cvt<R>(m.metric))) || (rc = b->upload(&b->fscale, cvt<R>(m.fscale))) ||
                (rc = b->upload(&b->frame, cvt<R>(m.frame))) || (rc = b->upload(&b->nbr, m.nbr)) ||

@@ -55,6 +55,11 @@ struct nexd_ctx {
     std::vector<int> fmask_host;
     double *metric = nullptr, *fscale = nullptr, *frame = nullptr, *jac = nullptr;
     int *nbr = nullptr, *ftype = nullptr;
+    double *AD = nullptr, *emet = nullptr;   // affine kernels (straight-sided meshes)
+    int *nbrt = nullptr;
+    bool affine = false;
+    nexd::OpsHost ops_host;
+    std::vector<double> affine_comb;         // AffineHost::comb of the mesh
     double *matc = nullptr, *emat = nullptr, *anel = nullptr, *pmlc = nullptr;
     double wl[nexd::NMB] = {0, 0, 0};
     std::vector<int> pmlcheck;
@@ -146,10 +151,22 @@ void drop_graph(nexd_ctx *c) {
 // stage launches (stage_launch.hpp: the kernels are instantiated in the
 // stage_*.hip translation units)
 // ---------------------------------------------------------------------------
-int nblocks(int order, int n, bool att, bool pml) { return nexd::stage_blocks<double>(order, n, att, pml); }
+int nblocks(const nexd_ctx *c, int n, bool att, bool pml) {
+    if (!c->affine) return nexd::stage_blocks<double>(c->cfg.order, n, att, pml);
+    const int order = c->cfg.order;
+    const int eb = nexd::affine_block<double>(order, att, pml, nexd::affine_shape_f64(order, att, pml, n)).eb;
+    return (n + eb - 1) / eb;
+}
 
-void dispatch_stage(int order, const StageArgs<double> &a, bool att, bool pml, hipStream_t s) {
-    if (a.scheme == NEXD_LSRK4) nexd::launch_stage<double, true, 0>(order, att, pml, a, s);
+void count_blocks(nexd_ctx *c) {
+    const bool att = c->cfg.attenuation != 0;
+    c->nblk_total = nblocks(c, c->n_plain, att, false) + nblocks(c, c->n_pml, att, true);
+}
+
+void dispatch_stage(const nexd_ctx *c, const StageArgs<double> &a, bool att, bool pml, hipStream_t s) {
+    const int order = c->cfg.order;
+    if (c->affine) nexd::launch_affine_f64(order, att, pml, a, s);
+    else if (a.scheme == NEXD_LSRK4) nexd::launch_stage<double, true, 0>(order, att, pml, a, s);
     else nexd::launch_stage<double, false, 0>(order, att, pml, a, s);
 }
 
@@ -253,6 +270,7 @@ StageArgs<double> base_args(nexd_ctx *c) {
     a.D = c->D; a.DK = nullptr; a.LT = c->LT; a.fmask = c->fmask;   // FP64: no contravariant form
     a.metric = c->metric; a.fscale = c->fscale; a.frame = c->frame; a.matc = c->matc;
     a.nbr = c->nbr; a.ftype = c->ftype; a.anel = c->anel;
+    a.AK = c->AD; a.emet = c->emet; a.fgeo = nullptr; a.nbrt = c->nbrt;
     for (int i = 0; i < nexd::NMB; ++i) a.wl[i] = c->wl[i];
     a.pmlc = c->pmlc;
     a.src_head = c->src_head; a.src_next = c->src_next; a.srctype = c->srctype;
@@ -330,13 +348,13 @@ void enqueue_step(nexd_ctx *c, const StepScratch &sc) {
         a.elist = c->elist_plain;
         a.nlist = c->n_plain;
         a.blk_energy = energy ? sc.blk_energy : nullptr;
-        dispatch_stage(c->cfg.order, a, att, false, c->stream);
+        dispatch_stage(c, a, att, false, c->stream);
         if (pml) {
             if (a.pml_compat && !a.recompute) dispatch_last_flux(c, qin, pin, sc.last_flux);
             a.elist = c->elist_pml;
             a.nlist = c->n_pml;
-            a.blk_energy = energy ? sc.blk_energy + nblocks(c->cfg.order, c->n_plain, att, false) : nullptr;
-            dispatch_stage(c->cfg.order, a, att, true, c->stream);
+            a.blk_energy = energy ? sc.blk_energy + nblocks(c, c->n_plain, att, false) : nullptr;
+            dispatch_stage(c, a, att, true, c->stream);
         }
         if (scheme == NEXD_EULER)
             (void)hipMemcpyAsync(c->q[0], c->q[1], sizeof(double) * 9 * c->nglob, hipMemcpyDeviceToDevice, c->stream);
@@ -364,8 +382,7 @@ int rebuild_lists(nexd_ctx *c) {
     if (c->n_pml) {
         HIPCHK(c, hipMemcpy(c->elist_pml, pmll.data(), sizeof(int) * pmll.size(), hipMemcpyHostToDevice));
     }
-    const bool att = c->cfg.attenuation != 0;
-    c->nblk_total = nblocks(c->cfg.order, c->n_plain, att, false) + nblocks(c->cfg.order, c->n_pml, att, true);
+    count_blocks(c);
     drop_graph(c);
     return 0;
 }
@@ -485,6 +502,12 @@ int nexd_create(const nexd_config *cfg, nexd_ctx **out) {
     return NEXD_OK;
 }
 
+// the affine kernels' operators, from the uploaded ones and the mesh
+static int put_affine_operators(nexd_ctx *c) {
+    return upload(c, &c->AD, nexd::mfma_affine_fragments_f64(nexd::affine_operators(c->ops_host.D, c->np, c->affine_comb),
+                                                             c->ops_host.LT, c->np, 4 * c->npf));
+}
+
 int nexd_upload_operators(nexd_ctx *c, const double *dr, const double *ds, const double *dt, const double *lift,
                           const double *mass, const int *fmask) {
     if (!c) return fail(c, NEXD_E_ARG, "null context");
@@ -497,6 +520,8 @@ int nexd_upload_operators(nexd_ctx *c, const double *dr, const double *ds, const
         (rc = upload(c, &c->fmask, o.fm)))
         return rc;
     c->fmask_host = o.fm;
+    c->ops_host = o;
+    if (c->affine && (rc = put_affine_operators(c))) return rc;
     c->have_ops = true;
     drop_graph(c);
     return NEXD_OK;
@@ -517,11 +542,24 @@ int nexd_upload_mesh(nexd_ctx *c, const int *ibool, const double *rx, const doub
     if (!err.empty())
         return err[0] == '!' ? fail(c, NEXD_E_UNSUPPORTED, err.substr(1)) : fail(c, NEXD_E_ARG, err);
     int rc;
-    if ((rc = upload(c, &c->metric, m.metric)) || (rc = upload(c, &c->jac, m.jac)) ||
-        (rc = upload(c, &c->fscale, m.fscale)) || (rc = upload(c, &c->frame, m.frame)) ||
-        (rc = upload(c, &c->nbr, m.nbr)) || (rc = upload(c, &c->ftype, m.ftype)))
+    // straight-sided meshes take the affine kernels (order 2 and up), every
+    // other the general ones
+    nexd::AffineHost ah;
+    const bool affine = c->cfg.order >= nexd::kAffMinOrder && nexd::affine_mesh(m, c->cfg.nelem, c->np, c->npf, true, ah);
+    if ((rc = upload(c, &c->jac, m.jac)) || (rc = upload(c, &c->fscale, m.fscale)) ||
+        (rc = upload(c, &c->frame, m.frame)))
         return rc;
+    if (affine) {
+        c->affine_comb = ah.comb;
+        if ((rc = put_affine_operators(c)) || (rc = upload(c, &c->emet, ah.emet)) || (rc = upload(c, &c->nbrt, ah.nbrt)))
+            return rc;
+    } else if ((rc = upload(c, &c->metric, m.metric)) || (rc = upload(c, &c->nbr, m.nbr)) ||
+               (rc = upload(c, &c->ftype, m.ftype))) {
+        return rc;
+    }
+    c->affine = affine;
     c->have_mesh = true;
+    count_blocks(c);
     drop_graph(c);
     return NEXD_OK;
 }
@@ -846,12 +884,12 @@ int nexd_time_stage_kernel(nexd_ctx *c, int list, int nrep, double *avg_ms, int 
     // launches: their values do not change the work.
     const bool att = c->cfg.attenuation != 0;
     // the last stage writes its energy partials, as in the time loop
-    double *en = energy_on(c) ? c->blk_energy + (list == 1 ? nblocks(c->cfg.order, c->n_plain, att, false) : 0)
+    double *en = energy_on(c) ? c->blk_energy + (list == 1 ? nblocks(c, c->n_plain, att, false) : 0)
                               : nullptr;
     auto one = [&](int irk) {
         stage_buffers(c, irk, a);
         a.blk_energy = a.last_stage ? en : nullptr;
-        dispatch_stage(c->cfg.order, a, att, list == 1, c->stream);
+        dispatch_stage(c, a, att, list == 1, c->stream);
     };
     stage_buffers(c, 1, a);
     if (list == 1 && a.recompute) dispatch_last_flux_rk2(c, c->last_flux);

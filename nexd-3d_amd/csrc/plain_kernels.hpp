@@ -109,9 +109,9 @@ struct StageArgs {
     int emat_stride;            // per-shot stride of emat (0: shared)
     const int *pml_on;          // [shot] 0 once a shot's PML is switched off; null: on
     // the affine kernels' operands (affine_kernels.hpp), FP32
-    const unsigned short *AK;   // [Dr|Ds|Dt|LIFT] in three bfloat16 parts [step][row tile][part][64][8]
+    const void *AK;             // [Dr|Ds|Dt|LIFT]: FP32 bfloat16 parts [step][row tile][part][64][8], FP64 [value][row tile][64]
     const R *emet;              // [nelem][12] metric (9) and padding
-    const R *fgeo;              // [nelem][4][4] normal, half the face scale
+    const R *fgeo;              // [nelem][4][4] normal, half the face scale (FP32)
     const int *nbrt;            // [nelem][4][NPF] neighbour node, -1 free, -2 absorbing
     // compensated state (float pairs hi + lo for the 9 wavefield components
     // and the receiver-element displacement); null when not compensated
@@ -129,57 +129,52 @@ struct StageArgs {
 // reference assembles as VT (src/timeloopMod.f90:262-271); free surfaces
 // apply diag(-2,0,0,-2,0,-2,0,0,0) between A+|A| and T^-1.
 // ---------------------------------------------------------------------------
+// Formed as traction and velocity jump and back: with T = sigma n, w1 = n.T,
+// w4 = s.T, w6 = t.T are rows 1, 4, 6 of T^-1 dq (w7, w8, w9 the velocity's;
+// the others meet zero columns of A+|A|), and the stress part of T z is
+//   n n^T z1 + (s s^T + t t^T) z2 + n c^T + c n^T,   c = s z4 + t z6.
+// lvl = lam vp / (lam + 2 mu) and irho = 1 / rho come with the material, p1 =
+// 1 / (vp rho) and p2 = 1 / (2 vs rho) are used with att; fs scales the result.
 template <typename R>
-__device__ __forceinline__ void upwind_flux(const R *fr, R vp, R vs, R rho, R lam, R mu, bool free,
-                                            const R dq[9], R out[9], R aout[6], bool att) {
+__device__ __forceinline__ void upwind_flux(const R *fr, R vp, R vs, R lam, R mu, R lvl, R irho, R p1, R p2, bool free,
+                                            R fs, const R dq[9], R *out, R *aout, bool att) {
     const R n0 = fr[0], n1 = fr[1], n2 = fr[2];
     const R s0 = fr[3], s1 = fr[4], s2 = fr[5];
     const R t0 = fr[6], t1 = fr[7], t2 = fr[8];
-    // rows 1, 4, 6, 7, 8, 9 of T^-1 dq (the others meet zero columns of A+|A|)
-    R w1 = n0 * n0 * dq[0] + n1 * n1 * dq[1] + n2 * n2 * dq[2] + 2 * n1 * n0 * dq[3] + 2 * n2 * n1 * dq[4] +
-           2 * n2 * n0 * dq[5];
-    R w4 = n0 * s0 * dq[0] + n1 * s1 * dq[1] + n2 * s2 * dq[2] + (n1 * s0 + n0 * s1) * dq[3] +
-           (n2 * s1 + n1 * s2) * dq[4] + (n2 * s0 + n0 * s2) * dq[5];
-    R w6 = n0 * t0 * dq[0] + n1 * t1 * dq[1] + n2 * t2 * dq[2] + (n1 * t0 + n0 * t1) * dq[3] +
-           (n2 * t1 + n1 * t2) * dq[4] + (n2 * t0 + n0 * t2) * dq[5];
-    R w7 = n0 * dq[6] + n1 * dq[7] + n2 * dq[8];
-    R w8 = s0 * dq[6] + s1 * dq[7] + s2 * dq[8];
-    R w9 = t0 * dq[6] + t1 * dq[7] + t2 * dq[8];
-    if (free) {
-        w1 = -2 * w1; w4 = -2 * w4; w6 = -2 * w6;
-        w7 = 0; w8 = 0; w9 = 0;
-    }
-    const R l2m = lam + 2 * mu;
-    const R z1 = vp * w1 - l2m * w7;
-    const R z2 = (lam * vp) / l2m * w1 - lam * w7;   // z3 == z2
-    const R z4 = vs * w4 - mu * w8;
-    const R z6 = vs * w6 - mu * w9;
-    const R irho = R(1) / rho;
-    const R z7 = -irho * w1 + vp * w7;
-    const R z8 = -irho * w4 + vs * w8;
-    const R z9 = -irho * w6 + vs * w9;
-    // T z (z5 == 0)
-    out[0] = n0 * n0 * z1 + (s0 * s0 + t0 * t0) * z2 + 2 * n0 * s0 * z4 + 2 * n0 * t0 * z6;
-    out[1] = n1 * n1 * z1 + (s1 * s1 + t1 * t1) * z2 + 2 * n1 * s1 * z4 + 2 * n1 * t1 * z6;
-    out[2] = n2 * n2 * z1 + (s2 * s2 + t2 * t2) * z2 + 2 * n2 * s2 * z4 + 2 * n2 * t2 * z6;
-    out[3] = n1 * n0 * z1 + (s1 * s0 + t1 * t0) * z2 + (n1 * s0 + n0 * s1) * z4 + (n1 * t0 + n0 * t1) * z6;
-    out[4] = n2 * n1 * z1 + (s2 * s1 + t2 * t1) * z2 + (n2 * s1 + n1 * s2) * z4 + (n2 * t1 + n1 * t2) * z6;
-    out[5] = n2 * n0 * z1 + (s2 * s0 + t2 * t0) * z2 + (n2 * s0 + n0 * s2) * z4 + (n2 * t0 + n0 * t2) * z6;
+    const R ft = free ? -2 * fs : fs, fv = free ? R(0) : fs;
+    const R T0 = ft * (dq[0] * n0 + dq[3] * n1 + dq[5] * n2);
+    const R T1 = ft * (dq[3] * n0 + dq[1] * n1 + dq[4] * n2);
+    const R T2 = ft * (dq[5] * n0 + dq[4] * n1 + dq[2] * n2);
+    const R v0 = fv * dq[6], v1 = fv * dq[7], v2 = fv * dq[8];
+    const R w1 = n0 * T0 + n1 * T1 + n2 * T2, w4 = s0 * T0 + s1 * T1 + s2 * T2, w6 = t0 * T0 + t1 * T1 + t2 * T2;
+    const R w7 = n0 * v0 + n1 * v1 + n2 * v2, w8 = s0 * v0 + s1 * v1 + s2 * v2, w9 = t0 * v0 + t1 * v1 + t2 * v2;
+    const R z1 = vp * w1 - (lam + 2 * mu) * w7;
+    const R z2 = lvl * w1 - lam * w7;   // z3 == z2
+    const R z4 = vs * w4 - mu * w8, z6 = vs * w6 - mu * w9;
+    const R z7 = vp * w7 - irho * w1, z8 = vs * w8 - irho * w4, z9 = vs * w9 - irho * w6;
+    const R c0 = s0 * z4 + t0 * z6, c1 = s1 * z4 + t1 * z6, c2 = s2 * z4 + t2 * z6;
+    const R m0 = n0 * z1, m1 = n1 * z1, m2 = n2 * z1;
+    out[0] = n0 * (m0 + 2 * c0) + (s0 * s0 + t0 * t0) * z2;
+    out[1] = n1 * (m1 + 2 * c1) + (s1 * s1 + t1 * t1) * z2;
+    out[2] = n2 * (m2 + 2 * c2) + (s2 * s2 + t2 * t2) * z2;
+    out[3] = n0 * (m1 + c1) + n1 * c0 + (s1 * s0 + t1 * t0) * z2;
+    out[4] = n1 * (m2 + c2) + n2 * c1 + (s2 * s1 + t2 * t1) * z2;
+    out[5] = n0 * (m2 + c2) + n2 * c0 + (s2 * s0 + t2 * t0) * z2;
     out[6] = n0 * z7 + s0 * z8 + t0 * z9;
     out[7] = n1 * z7 + s1 * z8 + t1 * z9;
     out[8] = n2 * z7 + s2 * z8 + t2 * z9;
     if (att) {
         // anelastic part: T(1:6,1:6) * A_anel * T^-1 dq
         // (src/waveMod.f90:146-159, src/timeloopMod.f90:270-271)
-        const R a1 = w1 / (vp * rho) - w7;
-        const R a4 = w4 / (2 * vs * rho) - w8 / 2;
-        const R a6 = w6 / (2 * vs * rho) - w9 / 2;
-        aout[0] = n0 * n0 * a1 + 2 * n0 * s0 * a4 + 2 * n0 * t0 * a6;
-        aout[1] = n1 * n1 * a1 + 2 * n1 * s1 * a4 + 2 * n1 * t1 * a6;
-        aout[2] = n2 * n2 * a1 + 2 * n2 * s2 * a4 + 2 * n2 * t2 * a6;
-        aout[3] = n1 * n0 * a1 + (n1 * s0 + n0 * s1) * a4 + (n1 * t0 + n0 * t1) * a6;
-        aout[4] = n2 * n1 * a1 + (n2 * s1 + n1 * s2) * a4 + (n2 * t1 + n1 * t2) * a6;
-        aout[5] = n2 * n0 * a1 + (n2 * s0 + n0 * s2) * a4 + (n2 * t0 + n0 * t2) * a6;
+        const R a1 = p1 * w1 - w7, a4 = p2 * w4 - w8 / 2, a6 = p2 * w6 - w9 / 2;
+        const R d0 = s0 * a4 + t0 * a6, d1 = s1 * a4 + t1 * a6, d2 = s2 * a4 + t2 * a6;
+        const R k0 = n0 * a1, k1 = n1 * a1, k2 = n2 * a1;
+        aout[0] = n0 * (k0 + 2 * d0);
+        aout[1] = n1 * (k1 + 2 * d1);
+        aout[2] = n2 * (k2 + 2 * d2);
+        aout[3] = n0 * (k1 + d1) + n1 * d0;
+        aout[4] = n1 * (k2 + d2) + n2 * d1;
+        aout[5] = n0 * (k2 + d2) + n2 * d0;
     }
 }
 
@@ -971,14 +966,16 @@ stage_kernel(StageArgs<R> a) {
                     for (int c = 0; c < 9; ++c) fr[c] = sFr[(fb * 4 + fi) * 9 + c];
                     const R *mc = sMc + fb * 5;
                     R fl[9], af[6];
-                    upwind_flux<R>(fr, mc[0], mc[1], mc[2], mc[3], mc[4], fty[i] == -1, dq, fl, af, ATT);
-                    const R sgn = fty[i] == -2 ? R(-1) : R(1);
+                    const R irho = R(1) / mc[2], lvl = mc[3] * mc[0] / (mc[3] + 2 * mc[4]);
+                    const R p1 = ATT ? irho / mc[0] : R(0), p2 = ATT ? R(0.5) * irho / mc[1] : R(0);
+                    const R fs = (fty[i] == -2 ? R(-0.5) : R(0.5)) * ffs[i];
+                    upwind_flux<R>(fr, mc[0], mc[1], mc[3], mc[4], lvl, irho, p1, p2, fty[i] == -1, fs, dq, fl, af, ATT);
                     R *dst = sF + fb * NFC * SFN + k;
 #pragma unroll
-                    for (int f = 0; f < 9; ++f) dst[f * SFN] = fvalid ? ffs[i] * (sgn * fl[f]) / 2 : R(0);
+                    for (int f = 0; f < 9; ++f) dst[f * SFN] = fvalid ? fl[f] : R(0);
                     if constexpr (ATT) {
 #pragma unroll
-                        for (int f = 0; f < 6; ++f) dst[(9 + f) * SFN] = fvalid ? ffs[i] * (sgn * af[f]) / 2 : R(0);
+                        for (int f = 0; f < 6; ++f) dst[(9 + f) * SFN] = fvalid ? af[f] : R(0);
                     }
                 }
             }
@@ -1106,20 +1103,20 @@ stage_kernel(StageArgs<R> a) {
             dq[f] = ft >= 0 ? qn - qo : qo;
         }
         const unsigned mb = nel * 8u * (unsigned)sizeof(R);
-        R mc[5], fr[9];
+        R mc[7], fr[9];
 #pragma unroll
-        for (int c = 0; c < 5; ++c) mc[c] = pload<BUF>(matc, mb, (unsigned)fe * 8 + c);
+        for (int c = 0; c < 7; ++c) mc[c] = c == 2 ? R(0) : pload<BUF>(matc, mb, (unsigned)fe * 8 + c);
 #pragma unroll
         for (int c = 0; c < 9; ++c) fr[c] = pload<BUF>(a.frame, nel * (unsigned)(36 * sizeof(R)), ((unsigned)fe * 4 + fi) * 9 + c);
         R fl[9], af[6];
-        upwind_flux<R>(fr, mc[0], mc[1], mc[2], mc[3], mc[4], ft == -1, dq, fl, af, ATT);
-        const R sgn = ft == -2 ? R(-1) : R(1);
-        const R fs = pload<BUF>(a.fscale, nel * (unsigned)(NFP * sizeof(R)), (unsigned)fe * NFP + k);
+        const R fs = (ft == -2 ? R(-0.5) : R(0.5)) * pload<BUF>(a.fscale, nel * (unsigned)(NFP * sizeof(R)), (unsigned)fe * NFP + k);
+        const R p1 = ATT ? mc[6] / mc[0] : R(0), p2 = ATT ? R(0.5) * mc[6] / mc[1] : R(0);
+        upwind_flux<R>(fr, mc[0], mc[1], mc[3], mc[4], mc[5], mc[6], p1, p2, ft == -1, fs, dq, fl, af, ATT);
 #pragma unroll
-        for (int f = 0; f < 9; ++f) dst[f * SFN] = fs * (sgn * fl[f]) / 2;
+        for (int f = 0; f < 9; ++f) dst[f * SFN] = fl[f];
         if constexpr (ATT) {
 #pragma unroll
-            for (int f = 0; f < 6; ++f) dst[(9 + f) * SFN] = fs * (sgn * af[f]) / 2;
+            for (int f = 0; f < 6; ++f) dst[(9 + f) * SFN] = af[f];
         }
     }
     __syncthreads();

@@ -47,3 +47,33 @@ def test_affine_and_general_route(order, att, pml):
                 assert rel_l2(got[name, tile][2], ref) <= 1e-4
                 assert np.array_equal(got[name, tile][0], got[name, tile][2])
         assert not np.array_equal(got["straight", 0][0], got["bent", 0][0])
+
+
+@pytest.mark.parametrize("order,cells", [(2, (3, 3, 3)), (2, (8, 7, 7)), (2, (12, 11, 11)), (3, (3, 3, 3)), (3, (8, 8, 8)),
+                                         (3, (12, 11, 11)), (4, (3, 3, 3)), (4, (5, 5, 5)), (4, (9, 8, 7)), (5, (3, 3, 3)),
+                                         (5, (6, 5, 5)), (5, (9, 8, 7))])
+@pytest.mark.parametrize("att,pml", [(False, 0), (True, 0), (False, 1), (True, 1)])
+def test_affine_and_general_route_fp64(order, cells, att, pml):
+    """FP64 single shots take the route for meshes whose metric is one
+    pattern times a constant per element to 1e-11; a change of 1e-10 in one
+    metric value takes the general kernels.  Mesh sizes on each side of the
+    lines between the block shapes; RK2, RK3 and the low-storage RK4 on the
+    smallest.  The two runs differ by that change and by 1e-11 of the metric:
+    1e-9 of the seismograms' (and energies') norm.
+    """
+    for timeint in (2, 3, 4) if cells == (3, 3, 3) else (2,):
+        p = problem.layered_box(*cells, order=order, nt=24, pml_cells=pml, nrec_side=2, attenuation=att, timeint=timeint)
+        rx = p.geom.rx.reshape(p.nelem, -1).copy()
+        rx[0, 0] += 1e-10 * np.abs(rx[0]).max()
+        bent = dataclasses.replace(p, geom=dataclasses.replace(p.geom, rx=rx.reshape(p.geom.rx.shape)))
+        got = []
+        for q in (p, bent):
+            print(f"[gpu affine fp64] N={order} {cells} att={att} pml={pml} timeint={timeint}", flush=True)
+            with capi.Context(layout.reference_arrays(q), energy=True) as ctx:
+                ctx.reset()
+                en = ctx.run(1, q.nt, want_energy=True)
+                got.append((ctx.seismograms(), np.asarray(en)))
+        assert np.linalg.norm(got[1][0]) > 0
+        for a, b in zip(*got):   # (the energy of a run without PML is zero)
+            assert np.linalg.norm(a - b) <= 1e-9 * np.linalg.norm(b)
+        assert not np.array_equal(got[0][0], got[1][0])
