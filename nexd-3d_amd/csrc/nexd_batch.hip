@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "../../include/nexd_gpu.h"
+#include "fill.hpp"
 #include "host_layout.hpp"
 #include "plain_kernels.hpp"
 #include "stage_launch.hpp"
@@ -510,37 +511,28 @@ struct Batch : BatchBase {
     int reset() {
         const size_t S = cfg.nshot;
         const R tiny = (R)(double)1e-24f;   // the reference's default-REAL 1e-24
+        nexd::Fill fill;
         for (int i = 0; i < 3; ++i) {
-            int rc = put(q[i], std::vector<R>(S * 9 * ng, tiny));
-            if (rc) return rc;
-            if (qlo[i] && (rc = put(qlo[i], std::vector<R>(S * 9 * ng, R(0))))) return rc;
+            fill.add(q[i], S * 9 * ng, tiny);
+            fill.add(qlo[i], S * 9 * ng, R(0));
         }
         if (cfg.attenuation)
-            for (int i = 0; i < 2; ++i) {
-                int rc = put(th[i], std::vector<R>(S * (i && recompute() ? 6 : 18) * ng, tiny));
-                if (rc) return rc;
-            }
+            for (int i = 0; i < 2; ++i) fill.add(th[i], S * (i && recompute() ? 6 : 18) * ng, tiny);
         if (cfg.pml)
-            for (int i = 0; i < 2; ++i) {
-                int rc = paux[i] ? put(paux[i], std::vector<R>(S * 27 * ng, R(0))) : 0;
-                if (rc) return rc;
-            }
-        if (qres) {
-            int rc;
-            if ((rc = put(qres, std::vector<R>(S * 9 * ng, R(0))))) return rc;
-            if (thres && (rc = put(thres, std::vector<R>(S * 18 * ng, R(0))))) return rc;
-            if (pres && (rc = put(pres, std::vector<R>(S * 27 * ng, R(0))))) return rc;
-        }
-        if (nslot) {
-            std::vector<R> t(S * nslot * 3 * np, tiny);
-            int rc;
-            if ((rc = put(u_slot, t)) || (rc = put(a_slot, t))) return rc;
-            if (u_slot_lo && (rc = put(u_slot_lo, std::vector<R>(S * nslot * 3 * np, R(0))))) return rc;
-        }
-        int rc = put(seis, std::vector<R>(S * 9 * cfg.nt * (cfg.nrec > 0 ? cfg.nrec : 1), R(0)));
-        if (rc) return rc;
-        if (energy && (rc = put(energy, std::vector<double>(S * cfg.nt, 0.0)))) return rc;
-        if ((rc = put(d_it, std::vector<int>(1, 0))) || (rc = put(d_done, std::vector<unsigned>(1, 0u)))) return rc;
+            for (int i = 0; i < 2; ++i) fill.add(paux[i], S * 27 * ng, R(0));
+        fill.add(qres, S * 9 * ng, R(0));
+        fill.add(thres, S * 18 * ng, R(0));
+        fill.add(pres, S * 27 * ng, R(0));
+        const size_t ns = S * nslot * 3 * np;
+        fill.add(u_slot, ns, tiny);
+        fill.add(a_slot, ns, tiny);
+        fill.add(u_slot_lo, ns, R(0));
+        fill.add(seis, S * 9 * cfg.nt * (cfg.nrec > 0 ? cfg.nrec : 1), R(0));
+        fill.add(energy, S * cfg.nt, 0.0);
+        fill.add(d_it, 1, 0);
+        fill.add(d_done, 1, 0u);
+        const hipError_t e = fill.run(cfg.device);
+        if (e != hipSuccess) return fail(NEXD_E_HIP, std::string("reset: ") + hipGetErrorString(e));
         step = 0;
         initialized = true;
         return 0;

@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "../../include/nexd_gpu.h"
+#include "fill.hpp"
 #include "host_layout.hpp"
 #include "plain_kernels.hpp"
 #include "stage_launch.hpp"
@@ -678,37 +679,24 @@ int nexd_reset(nexd_ctx *c) {
     const size_t ng = c->nglob;
     // the reference assigns the default-REAL literal 1e-24 (src/timeloopMod.f90:184-195)
     const double tiny_v = (double)1e-24f;
-    std::vector<double> tiny(9 * ng, tiny_v);
-    for (int i = 0; i < 3; ++i) HIPCHK(c, hipMemcpy(c->q[i], tiny.data(), sizeof(double) * 9 * ng, hipMemcpyHostToDevice));
-    if (c->cfg.attenuation) {
-        std::vector<double> t18(18 * ng, tiny_v);
-        for (int i = 0; i < 2; ++i)
-            HIPCHK(c, hipMemcpy(c->th[i], t18.data(), sizeof(double) * (i && recompute(c) ? 6 : 18) * ng, hipMemcpyHostToDevice));
-    }
-    if (c->cfg.pml) {
-        std::vector<double> z(27 * ng, 0.0);
-        for (int i = 0; i < 2; ++i)
-            if (c->paux[i]) HIPCHK(c, hipMemcpy(c->paux[i], z.data(), sizeof(double) * 27 * ng, hipMemcpyHostToDevice));
-    }
-    if (c->u_full) HIPCHK(c, hipMemcpy(c->u_full, tiny.data(), sizeof(double) * 3 * ng, hipMemcpyHostToDevice));
-    if (c->qres) {
-        const std::vector<double> z(27 * ng, 0.0);
-        HIPCHK(c, hipMemcpy(c->qres, z.data(), sizeof(double) * 9 * ng, hipMemcpyHostToDevice));
-        if (c->thres) HIPCHK(c, hipMemcpy(c->thres, z.data(), sizeof(double) * 18 * ng, hipMemcpyHostToDevice));
-        if (c->pres) HIPCHK(c, hipMemcpy(c->pres, z.data(), sizeof(double) * 27 * ng, hipMemcpyHostToDevice));
-    }
-    if (c->nslot) {
-        std::vector<double> t(3 * (size_t)c->nslot * c->np, tiny_v);
-        HIPCHK(c, hipMemcpy(c->u_slot, t.data(), sizeof(double) * t.size(), hipMemcpyHostToDevice));
-        HIPCHK(c, hipMemcpy(c->a_slot, t.data(), sizeof(double) * t.size(), hipMemcpyHostToDevice));
-    }
-    std::vector<double> zs((size_t)9 * c->cfg.nt * (c->cfg.nrec > 0 ? c->cfg.nrec : 1), 0.0);
-    HIPCHK(c, hipMemcpy(c->seis, zs.data(), sizeof(double) * zs.size(), hipMemcpyHostToDevice));
-    std::vector<double> ze(c->cfg.nt, 0.0);
-    HIPCHK(c, hipMemcpy(c->energy, ze.data(), sizeof(double) * ze.size(), hipMemcpyHostToDevice));
-    int zero = 0;
-    HIPCHK(c, hipMemcpy(c->d_it, &zero, sizeof(int), hipMemcpyHostToDevice));
-    HIPCHK(c, hipMemcpy(c->d_done, &zero, sizeof(unsigned), hipMemcpyHostToDevice));
+    nexd::Fill fill;
+    for (int i = 0; i < 3; ++i) fill.add(c->q[i], 9 * ng, tiny_v);
+    if (c->cfg.attenuation)
+        for (int i = 0; i < 2; ++i) fill.add(c->th[i], (i && recompute(c) ? 6 : 18) * ng, tiny_v);
+    if (c->cfg.pml)
+        for (int i = 0; i < 2; ++i) fill.add(c->paux[i], 27 * ng, 0.0);
+    fill.add(c->u_full, 3 * ng, tiny_v);
+    fill.add(c->qres, 9 * ng, 0.0);
+    fill.add(c->thres, 18 * ng, 0.0);
+    fill.add(c->pres, 27 * ng, 0.0);
+    const size_t ns = 3 * (size_t)c->nslot * c->np;
+    fill.add(c->u_slot, ns, tiny_v);
+    fill.add(c->a_slot, ns, tiny_v);
+    fill.add(c->seis, (size_t)9 * c->cfg.nt * (c->cfg.nrec > 0 ? c->cfg.nrec : 1), 0.0);
+    fill.add(c->energy, (size_t)c->cfg.nt, 0.0);
+    fill.add(c->d_it, 1, 0);
+    fill.add(c->d_done, 1, 0u);
+    HIPCHK(c, fill.run(c->cfg.device));
     c->step = 0;
     c->initialized = true;
     return NEXD_OK;
