@@ -42,26 +42,18 @@ def log(msg):
     print(msg, file=sys.stderr, flush=True)
 
 
-def b_alg(np_, nv, w, r, nshot=1):
-    """Algorithmic HBM bytes of one element-stage for nshot shots of one
-    element: w*Np*nv*(2+r) per shot (read and write each wavefield, memory
-    variable and PML auxiliary once, plus the RK base on stages that read
-    it, r = 1), plus 54 reals of element metadata (9 affine metric terms, 4
-    fscale, 36 face frame components, 5 material values) and 48 bytes of
-    connectivity, shared by the shots of a launch (one geometry, one
-    material set)."""
-    return nshot * w * np_ * nv * (2 + r) + 54 * w + 48
-
-
-def b_alg_stage_mean(np_, nv, w, nrk=2, nshot=1):
-    """b_alg averaged over the nrk stages of a step: stage 1 reads no RK
-    base, the later ones do."""
-    return (b_alg(np_, nv, w, 0, nshot) + (nrk - 1) * b_alg(np_, nv, w, 1, nshot)) / nrk
-
-
-# wavefield values per node of a PML element with attenuation: 9 fields,
-# 18 memory variables, 27 PML auxiliaries
-NV_PML_ATT = 9 + 18 + 27
+def b_alg_rk2(np_, w, compensated=False, nshot=1):
+    """Mean algorithmic HBM bytes of one element-stage of a TVD RK2 step of PML
+    elements with attenuation, for nshot shots of one element.  Stage 2
+    repeats the stage-1 update of the element-local values, so stage 1 reads
+    54 values of a node (9 fields, 18 memory variables, 27 PML auxiliaries)
+    and writes 15 (9 fields, 6 rates common to the memory variables), stage 2
+    reads 69 (stage-1 and step-start fields, 6, 18, 27) and writes 54; the low
+    parts of the compensated fields add 9 to each read and write of them.
+    54 reals of element metadata (metric, face scales and frames, material) and
+    48 bytes of connectivity are shared by the shots of a launch."""
+    values = 192 + (45 if compensated else 0)
+    return nshot * w * np_ * values / 2 + 54 * w + 48
 
 
 def traffic_file(order: int) -> str:
@@ -92,7 +84,7 @@ def pmc_summary(fetch_csv, write_csv, copy_fetch_csv, copy_write_csv):
     f, wr = per_kernel(fetch_csv, "FETCH_SIZE"), per_kernel(write_csv, "WRITE_SIZE")
     out = {"fetch_scale": fs, "write_scale": ws, "kernels": {}}
     for name in f:
-        if "stage_kernel" not in name or name not in wr:
+        if not ("stage_kernel" in name or "affine_kernel" in name) or name not in wr:
             continue
         rd = sum(f[name]) / len(f[name]) * 1024 * fs
         wt = sum(wr[name]) / len(wr[name]) * 1024 * ws
@@ -412,11 +404,11 @@ def main():
     nsteps_all = args.warmup + args.steps
 
     np_ = p.ref.np_
-    bpe64 = b_alg_stage_mean(np_, NV_PML_ATT, 8)                    # one shot per launch
+    bpe64 = b_alg_rk2(np_, 8)                    # one shot per launch
     # per element-shot; the compensated sum also reads and writes the low
     # parts of the 9 fields (and reads the RK base's on stage 2)
-    bpe32 = b_alg_stage_mean(np_, NV_PML_ATT + 9, 4, nshot=sb.nshot) / sb.nshot
-    bpe32_plain = b_alg_stage_mean(np_, NV_PML_ATT, 4, nshot=sb.nshot) / sb.nshot
+    bpe32 = b_alg_rk2(np_, 4, True, nshot=sb.nshot) / sb.nshot
+    bpe32_plain = b_alg_rk2(np_, 4, nshot=sb.nshot) / sb.nshot
 
     # ---- FP64 plain path (the drop-in), shot 0 ------------------------------
     fp64 = None
@@ -481,11 +473,12 @@ def main():
     if os.path.exists(tfile):
         tf = json.load(open(tfile))
         if tf.get("workload") == workload_key:
-            for name, v in tf["kernels"].items():
-                if f"<{args.order}, true, true, float," in name:
-                    traffic = v["bytes_per_launch"]
-                elif f"<{args.order}, true, true, double," in name:
-                    traffic64 = v["bytes_per_launch"]
+            # the stages have kernels of their own: the mean over them
+            def mean_bytes(kind):
+                k = [v["bytes_per_launch"] for n, v in tf["kernels"].items() if f"<{args.order}, true, true, {kind}," in n]
+                return sum(k) / len(k) if k else None
+
+            traffic, traffic64 = mean_bytes("float"), mean_bytes("double")
     out = {
         "metric": "DOF-updates/s on 1 GPU: FP64 plain vs FP32 batched at ≤1e-4 seismogram L2",
         "value": value32,
@@ -517,12 +510,12 @@ def main():
                    "accuracy": accuracy},
         "roofline": {"bound": "hbm", "achieved": achieved32, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved32 / HBM_PEAK_GBS, "traffic": traffic,
-                     "kernel": f"stage_kernel<{args.order},ATT,PML,f32> (PML elements, all shots, compensated; mean "
+                     "kernel": f"affine_kernel<{args.order},ATT,PML,f32> (PML elements, all shots, compensated; mean "
                                f"over the 2 RK stages, energy partials on the second)",
                      "bytes_per_element_shot": bpe32,
-                     "bytes_model": "w*Np*63*(2+r) per element-shot (9 fields with their low parts, 18 memory "
-                                    "variables, 27 PML auxiliaries; r: RK base read on stage 2) + (54*w + 48) per "
-                                    "element shared by the shots",
+                     "bytes_model": "w*Np*237/2 per element-shot and stage (9 fields with their low parts, 18 memory "
+                                    "variables or their 6 common rates, 27 PML auxiliaries; stage 2 repeats stage 1's "
+                                    "element-local update) + (54*w + 48) per element shared by the shots",
                      "algorithmic_bytes_per_launch": bpe32 * n32_pml * sb.nshot,
                      "avg_launch_ms": ms32_pml, "elements_per_launch": n32_pml, "shots_per_launch": sb.nshot,
                      "traffic_source": os.path.relpath(tfile, ROOT) if traffic else None,
