@@ -38,17 +38,12 @@
 //     where the FP32 instruction takes 256, and with fewer roundings: that one
 //     rounds after every product (rms error 2.5 eps R at 64 products, R the
 //     root of their squares' sum), this one 0.8 with the five small products in
-//     a sum of their own;
-//   - what would round the same way at every step, and so add up as a phase
-//     error of the waves, is kept: the step and the material of the volume term
-//     enter with their rounding as a low part of dt (step_of), the flux is formed
-//     in double from double geometry and materials (affine_flux).  The flux in
-//     double is 1 to 4 % of a run.
-// The seismograms' error against 64 bits, over random sizes, orders 2 to 5, with
-// and without attenuation and PML, is 0.02 to 1.2 of the general kernel's, 0.6 at
-// the median; one FP32 chain over the whole product would give 1.3 to 1.8.
+//     a sum of their own.  The seismograms' error against 64 bits, over random
+//     sizes, orders 2 to 5, with and without attenuation and PML, is 0.2 to 1.1
+//     of the general kernel's (one FP32 chain over the whole product would give
+//     1.3 to 1.8).
 // Measured against the general kernel, per stage: N = 3 elastic, 64 shots on
-// 3,072 tets 360 -> 278 us; elastic single shots N = 2, 3, 4, 5 33 -> 26, 44 ->
+// 3,072 tets 360 -> 269 us; elastic single shots N = 2, 3, 4, 5 33 -> 26, 44 ->
 // 29, 68 -> 37, 195 -> 95 us; N = 4 with attenuation and PML, 8 shots, stages
 // 1 and 2 1,466 -> 1,294 and 2,174 -> 1,953 us (3.2 and 3.5 TB/s of traffic; a
 // large copy reaches 4.7).  Vector instructions are now 42 to 53 % of the time,
@@ -78,7 +73,6 @@
 namespace nexd {
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
-typedef double f64x4_t __attribute__((ext_vector_type(4)));
 typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 
@@ -111,7 +105,7 @@ __device__ __forceinline__ void split3(const float (&v)[8], bf16x8_t (&b)[3]) {
 }
 
 // values per element staged in LDS: the metric (9), the coefficients of the
-// columns (7, see column_terms) and (FP64) the material terms of the flux
+// columns (7, see column_terms) and the material terms of the flux
 constexpr int kAffElem = 23;
 enum AffElem { AE_MET = 0, AE_COEF = 9, AE_VP = 16, AE_VS, AE_LAM, AE_MU, AE_LVL, AE_P1, AE_P2 };
 
@@ -123,47 +117,42 @@ enum AffElem { AE_MET = 0, AE_COEF = 9, AE_VP = 16, AE_VS, AE_LAM, AE_MU, AE_LVL
 //   z1 = vp T_n - (lam + 2 mu) v_n,  z2 = lam vp/(lam + 2 mu) T_n - lam v_n,  z7 = -T_n / rho + vp v_n
 // (s s^T + t t^T = I - n n^T, so the tangents drop out), and of the anelastic
 // part, a1 = T_n/(vp rho) - v_n, c = T_t/(2 vs rho) - v_t/2: n n^T a1 + n c^T + c n^T.
-// In double, from double geometry and materials (el: vp, vs, lam, mu, lam vp/(lam +
-// 2 mu), 1/rho, p1, p2): rounded to single precision they act like another wave
-// speed (normals 2.6e-6, face scales 4.3e-6, material 1e-6 to 5e-6 of the
-// seismograms after 101 to 147 steps at N = 2), and with LIFT not rounded here
-// nothing would offset them.
 template <bool ATT>
-__device__ __forceinline__ void affine_flux(double n0, double n1, double n2, double fs, const double *el,
+__device__ __forceinline__ void affine_flux(float n0, float n1, float n2, float fs, const float *el, float coef_ef3,
                                             bool free, const float dq[9], float out[ATT ? 15 : 9]) {
-    const double vp = el[0], vs = el[1], lam = el[2], mu = el[3], lvl = el[4], ef3 = -el[5];
-    const double ft = free ? -2. * fs : fs, fv = free ? 0. : fs;
-    const double T0 = ft * (dq[0] * n0 + dq[3] * n1 + dq[5] * n2);
-    const double T1 = ft * (dq[3] * n0 + dq[1] * n1 + dq[4] * n2);
-    const double T2 = ft * (dq[5] * n0 + dq[4] * n1 + dq[2] * n2);
-    const double v0 = fv * dq[6], v1 = fv * dq[7], v2 = fv * dq[8];
-    const double Tn = T0 * n0 + T1 * n1 + T2 * n2, vn = v0 * n0 + v1 * n1 + v2 * n2;
-    const double t0 = T0 - n0 * Tn, t1 = T1 - n1 * Tn, t2 = T2 - n2 * Tn;
-    const double u0 = v0 - n0 * vn, u1 = v1 - n1 * vn, u2 = v2 - n2 * vn;
-    const double z1 = vp * Tn - (lam + 2. * mu) * vn, z2 = lvl * Tn - lam * vn, dz = z1 - z2;
-    const double a0 = vs * t0 - mu * u0, a1 = vs * t1 - mu * u1, a2 = vs * t2 - mu * u2;
-    const double m0 = n0 * dz, m1 = n1 * dz, m2 = n2 * dz;
-    out[0] = (float)(n0 * (m0 + 2. * a0) + z2);
-    out[1] = (float)(n1 * (m1 + 2. * a1) + z2);
-    out[2] = (float)(n2 * (m2 + 2. * a2) + z2);
-    out[3] = (float)(n0 * (m1 + a1) + n1 * a0);
-    out[4] = (float)(n1 * (m2 + a2) + n2 * a1);
-    out[5] = (float)(n0 * (m2 + a2) + n2 * a0);
-    const double z7 = ef3 * Tn + vp * vn;
-    out[6] = (float)(n0 * z7 + (ef3 * t0 + vs * u0));
-    out[7] = (float)(n1 * z7 + (ef3 * t1 + vs * u1));
-    out[8] = (float)(n2 * z7 + (ef3 * t2 + vs * u2));
+    const float vp = el[AE_VP], vs = el[AE_VS], lam = el[AE_LAM], mu = el[AE_MU], lvl = el[AE_LVL];
+    const float ft = free ? -2.f * fs : fs, fv = free ? 0.f : fs;
+    const float T0 = ft * (dq[0] * n0 + dq[3] * n1 + dq[5] * n2);
+    const float T1 = ft * (dq[3] * n0 + dq[1] * n1 + dq[4] * n2);
+    const float T2 = ft * (dq[5] * n0 + dq[4] * n1 + dq[2] * n2);
+    const float v0 = fv * dq[6], v1 = fv * dq[7], v2 = fv * dq[8];
+    const float Tn = T0 * n0 + T1 * n1 + T2 * n2, vn = v0 * n0 + v1 * n1 + v2 * n2;
+    const float t0 = T0 - n0 * Tn, t1 = T1 - n1 * Tn, t2 = T2 - n2 * Tn;
+    const float u0 = v0 - n0 * vn, u1 = v1 - n1 * vn, u2 = v2 - n2 * vn;
+    const float z1 = vp * Tn - (lam + 2.f * mu) * vn, z2 = lvl * Tn - lam * vn, dz = z1 - z2;
+    const float a0 = vs * t0 - mu * u0, a1 = vs * t1 - mu * u1, a2 = vs * t2 - mu * u2;
+    const float m0 = n0 * dz, m1 = n1 * dz, m2 = n2 * dz;
+    out[0] = n0 * (m0 + 2.f * a0) + z2;
+    out[1] = n1 * (m1 + 2.f * a1) + z2;
+    out[2] = n2 * (m2 + 2.f * a2) + z2;
+    out[3] = n0 * (m1 + a1) + n1 * a0;
+    out[4] = n1 * (m2 + a2) + n2 * a1;
+    out[5] = n0 * (m2 + a2) + n2 * a0;
+    const float z7 = coef_ef3 * Tn + vp * vn;   // coef_ef3 = -1/rho
+    out[6] = n0 * z7 + (coef_ef3 * t0 + vs * u0);
+    out[7] = n1 * z7 + (coef_ef3 * t1 + vs * u1);
+    out[8] = n2 * z7 + (coef_ef3 * t2 + vs * u2);
     if constexpr (ATT) {
-        const double p1 = el[6], p2 = el[7];   // 1/(vp rho), 1/(2 vs rho)
-        const double b = p1 * Tn - vn;
-        const double c0 = p2 * t0 - 0.5 * u0, c1 = p2 * t1 - 0.5 * u1, c2 = p2 * t2 - 0.5 * u2;
-        const double k0 = n0 * b, k1 = n1 * b, k2 = n2 * b;
-        out[9] = (float)(n0 * (k0 + 2. * c0));
-        out[10] = (float)(n1 * (k1 + 2. * c1));
-        out[11] = (float)(n2 * (k2 + 2. * c2));
-        out[12] = (float)(n0 * (k1 + c1) + n1 * c0);
-        out[13] = (float)(n1 * (k2 + c2) + n2 * c1);
-        out[14] = (float)(n0 * (k2 + c2) + n2 * c0);
+        const float p1 = el[AE_P1], p2 = el[AE_P2];   // 1/(vp rho), 1/(2 vs rho)
+        const float b = p1 * Tn - vn;
+        const float c0 = p2 * t0 - 0.5f * u0, c1 = p2 * t1 - 0.5f * u1, c2 = p2 * t2 - 0.5f * u2;
+        const float k0 = n0 * b, k1 = n1 * b, k2 = n2 * b;
+        out[9] = n0 * (k0 + 2.f * c0);
+        out[10] = n1 * (k1 + 2.f * c1);
+        out[11] = n2 * (k2 + 2.f * c2);
+        out[12] = n0 * (k1 + c1) + n1 * c0;
+        out[13] = n1 * (k2 + c2) + n2 * c1;
+        out[14] = n0 * (k2 + c2) + n2 * c0;
     }
 }
 
@@ -249,7 +238,7 @@ struct AffShape {
         if (cap < eb) eb = cap;
         // with the PML one wave at least is left to the face term
         if (PML && eb * NP > 192 && 192 / NP >= 2) eb = 192 / NP;
-        while (eb > 1 && lds_reals(eb) * 4 + 72 * eb + 64 > 160 * 1024 / BPC) --eb;
+        while (eb > 1 && lds_reals(eb) * 4 + 8 * eb + 64 > 160 * 1024 / BPC) --eb;
         return eb;
     }
     static constexpr int EB = pick_eb();
@@ -292,7 +281,6 @@ affine_kernel(StageArgs<R> a) {
     // few loads of a thread come out 2 % faster as global ones
     constexpr bool BUF = PML || ATT;
     __shared__ __align__(16) R lds[S::LDS];
-    __shared__ double sD[F64 ? 1 : EB * 8];   // FP32: the flux's materials
     R *sQ = lds;                        // [9][NT]
     R *sC = lds + 9 * NT;               // [3][9][NT] contravariant fluxes (PML)
     R *sF = lds + S::OFF_F;             // [EB][NCOL][SFN] face values
@@ -322,7 +310,7 @@ affine_kernel(StageArgs<R> a) {
     const int e = valid ? a.elist[idx] : 0;
     const unsigned g32 = (unsigned)e * NP + j;
     const size_t g = (size_t)e * NP + j;
-    const R dt = a.dt_elem ? a.dt_elem[e] : a.dt, dt_lo = F64 ? R(0) : (a.dt_elem ? a.dt_elem_lo[e] : a.dt_lo);
+    const R dt = a.dt_elem ? a.dt_elem[e] : a.dt;
 
     // Element constants into LDS.  Elements past the end of the list take
     // element 0's; their values are finite and never stored.
@@ -339,20 +327,15 @@ affine_kernel(StageArgs<R> a) {
             for (int k = 0; k < 9; ++k) el[AE_MET + k] = met[k];
             el[AE_COEF + 0] = -(lam + R(2) * mu); el[AE_COEF + 1] = -lam; el[AE_COEF + 2] = -mu; el[AE_COEF + 3] = -irho;
             el[AE_COEF + 4] = R(0); el[AE_COEF + 5] = -R(1); el[AE_COEF + 6] = -R(0.5);
-            if constexpr (F64) { el[AE_VP] = vp; el[AE_VS] = vs; el[AE_LAM] = lam; el[AE_MU] = mu; el[AE_LVL] = lvl; }
-            if constexpr (!F64) {
-                const double *md = a.matd + (size_t)shot * a.mat_stride + (size_t)ee * 8;
-#pragma unroll
-                for (int k = 0; k < 8; ++k) sD[i * 8 + k] = md[k];
-            }
-            if constexpr (F64 && ATT) { el[AE_P1] = irho / vp; el[AE_P2] = R(0.5) * irho / vs; }
+            el[AE_VP] = vp; el[AE_VS] = vs; el[AE_LAM] = lam; el[AE_MU] = mu; el[AE_LVL] = lvl;
+            if constexpr (ATT) { el[AE_P1] = irho / vp; el[AE_P2] = R(0.5) * irho / vs; }
         }
     };
 
     // The face nodes of thread th of the face term: what does not depend on
     // this block's own values, the neighbour traces among it
     R fq[FIT][9];
-    f64x4_t fg[F64 ? 1 : FIT];
+    f32x4_t fg[F64 ? 1 : FIT];
     R ffr[F64 ? FIT : 1][9], ffs[F64 ? FIT : 1];
     int fnb[FIT], fown[FIT];
     auto face_load = [&](int th) {
@@ -371,7 +354,7 @@ affine_kernel(StageArgs<R> a) {
 #pragma unroll
                 for (int c = 0; c < 9; ++c) ffr[i][c] = a.frame[((size_t)fe[i] * 4 + k / NPF) * 9 + c];
             } else {
-                fg[i] = *reinterpret_cast<const f64x4_t *>(a.fgeo + ((size_t)fe[i] * 4 + k / NPF) * 4);
+                fg[i] = *reinterpret_cast<const f32x4_t *>(a.fgeo + ((size_t)fe[i] * 4 + k / NPF) * 4);
             }
             fown[i] = fb * NP + a.fmask[k];
         }
@@ -403,8 +386,8 @@ affine_kernel(StageArgs<R> a) {
                     upwind_flux<R>(ffr[i], el[AE_VP], el[AE_VS], el[AE_LAM], el[AE_MU], el[AE_LVL], -el[AE_COEF + 3],
                                    el[AE_P1], el[AE_P2], fnb[i] == -1, fs, dq, fl, fl + (ATT ? 9 : 0), ATT);
                 } else {
-                    const double fs = fvalid ? (fnb[i] == -1 ? -fg[i][3] : fg[i][3]) : 0.0;
-                    affine_flux<ATT>(fg[i][0], fg[i][1], fg[i][2], fs, sD + fb * 8, fnb[i] == -1, dq, fl);
+                    const R fs = fvalid ? (fnb[i] == -1 ? -fg[i][3] : fg[i][3]) : R(0);
+                    affine_flux<ATT>(fg[i][0], fg[i][1], fg[i][2], fs, el, el[AE_COEF + 3], fnb[i] == -1, dq, fl);
                 }
                 R *dst = sF + fb * NCOL * SFN + k;
 #pragma unroll
@@ -569,6 +552,7 @@ affine_kernel(StageArgs<R> a) {
         // and the operator's fragments of the wave's row tiles load PREF values
         // ahead.
         constexpr int RW = S::RW, RG = S::RG, CW = S::CW, CG = S::CG, KT = S::KT, PREF = 12 / RW;
+        typedef double f64x4_t __attribute__((ext_vector_type(4)));
         const int r0 = (w % RG) * RW, c0 = w / RG;
         const double *ak = reinterpret_cast<const double *>(a.AK) + lane;
         double af[PREF][RW];
@@ -774,15 +758,10 @@ affine_kernel(StageArgs<R> a) {
 
     // ---- node threads: memory variables, sources, Runge-Kutta update -------
     R th[ATT ? 18 : 1], thb[ATT && RC == 0 ? 18 : 1], gi[ATT && RC == 2 ? 6 : 1], avc[ATT ? 9 : 1];
-    R qb[9], alo[9], blo[9], mcor[3];
+    R qb[9], alo[9], blo[9];
     const bool comp = a.qlo_out != nullptr;
     const unsigned nel = (unsigned)(ng / NP);
     if (node_thr) {
-        if constexpr (!F64) {
-            const R *mc = a.mcor + (size_t)shot * a.emat_stride * 2 + (size_t)e * 4;
-#pragma unroll
-            for (int k = 0; k < 3; ++k) mcor[k] = mc[k];
-        }
         if constexpr (ATT) {
             const R *thin = a.thin + (size_t)shot * 18 * ng;
             const R *av = a.anel + (size_t)shot * a.anel_stride;
@@ -868,21 +847,13 @@ affine_kernel(StageArgs<R> a) {
             }
         }
         if (valid) add_sources<NP>(a, shot, j, src_first, it_step, rhs);
-        // dt times the rate of field f, rounded once; FP32 with the low part of
-        // the step and the material's
-        R low[3];
-        if constexpr (!F64) {
-#pragma unroll
-            for (int k = 0; k < 3; ++k) low[k] = fma_r(dt, mcor[k], dt_lo);
-        }
-        auto step_of = [&](R r, int f) { return F64 ? r * dt : fma_r(r, dt, r * low[f / 3]); };
         if (!LS && comp) {
             const int scheme = RC ? 2 : a.scheme, irk = RC ? RC : a.irk;
 #pragma unroll
             for (int f = 0; f < 9; ++f) {
                 R lo;
                 const R b = RC == 1 ? qs[f] : qb[f], bl = RC == 1 ? alo[f] : blo[f];
-                rk_combine_comp<R>(scheme, irk, qs[f], alo[f], b, bl, step_of(rhs[f], f), R(1), a.w13, a.w23, qnew[f], lo);
+                rk_combine_comp<R>(scheme, irk, qs[f], alo[f], b, bl, rhs[f], dt, a.w13, a.w23, qnew[f], lo);
                 if (valid) {
                     pstore<BUF>(qout + f * ng, pnb, g32, qnew[f]);
                     pstore<BUF>(a.qlo_out + ((size_t)shot * 9 + f) * ng, pnb, g32, lo);
@@ -892,7 +863,7 @@ affine_kernel(StageArgs<R> a) {
 #pragma unroll
             for (int f = 0; f < 9; ++f) {
                 if constexpr (RC == 1) qb[f] = R(0);
-                qnew[f] = rk_update<R, LS, WEIGHTED, RC>(rs, qs[f], qb[f], step_of(rhs[f], f), R(1));
+                qnew[f] = rk_update<R, LS, WEIGHTED, RC>(rs, qs[f], qb[f], rhs[f], dt);
             }
             if (valid) {
 #pragma unroll

@@ -120,7 +120,10 @@ inline double bf16_value(unsigned short b) {
 // operand supplies values of its own: entry i of step st is value s = 8 st + i
 // of lane group l/16, for s = 3 ks + o (ks < ceil(Np/4)) operator o at node
 // 4ks + l/16, then LIFT at face nodes 4ks + l/16; zero beyond Np and past the
-// last value.
+// last value.  LIFT enters as the general FP32 kernel has it, rounded to single
+// precision: its rounding and those of face scales, normals, material and step
+// act like another wave speed (4.7e-6, 4.3e-6, 2.6e-6, 0.9e-6 and 1.6e-6 of the
+// seismograms after 101 steps at N = 2), and partly offset each other.
 inline std::vector<unsigned short> mfma_affine_fragments(const std::vector<double> &D, const std::vector<double> &LT,
                                                          int np, int nfp) {
     const int nt = (np + 15) / 16, ksv = 3 * ((np + 3) / 4), kt = ksv + nfp / 4, ns = (kt + 7) / 8;
@@ -130,7 +133,7 @@ inline std::vector<unsigned short> mfma_affine_fragments(const std::vector<doubl
             for (int l = 0; l < 64; ++l) {
                 const int node = 16 * rt + l % 16, k = 4 * (s < ksv ? s / 3 : s - ksv) + l / 16;
                 if (node >= np || (s < ksv && k >= np)) continue;
-                double x = s < ksv ? D[((size_t)(s % 3) * np + node) * np + k] : LT[(size_t)k * np + node];
+                double x = s < ksv ? D[((size_t)(s % 3) * np + node) * np + k] : (double)(float)LT[(size_t)k * np + node];
                 for (int p = 0; p < 3; ++p) {
                     const unsigned short b = bf16_bits(x);
                     out[((((size_t)(s / 8) * nt + rt) * 3 + p) * 64 + l) * 8 + s % 8] = b;

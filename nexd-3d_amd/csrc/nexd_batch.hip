@@ -57,16 +57,14 @@ struct Batch : BatchBase {
     R *jac = nullptr;
     unsigned short *AK = nullptr;                        // affine kernels (straight-sided meshes): FP32, FP64 operators
     double *AD = nullptr;
-    R *emet = nullptr;
-    double *fgeo = nullptr;
+    R *emet = nullptr, *fgeo = nullptr;
     int *nbrt = nullptr;
     bool affine = false;
     nexd::OpsHost ops_host;
     std::vector<double> affine_comb;   // AffineHost::comb of the mesh
     int *fmask = nullptr, *nbr = nullptr, *ftype = nullptr;
     std::vector<int> fmask_host;
-    R *matc = nullptr, *anel = nullptr, *pmlc = nullptr, *emat = nullptr, *mcor = nullptr;
-    double *matd = nullptr;
+    R *matc = nullptr, *anel = nullptr, *pmlc = nullptr, *emat = nullptr;
     double wl[nexd::NMB] = {0, 0, 0};
     std::vector<int> pmlcheck;
     int *elist_plain = nullptr, *elist_pml = nullptr;
@@ -83,7 +81,6 @@ struct Batch : BatchBase {
     int nblk_total = 0;
     int tile = 0;                             // block shape of the stage launches (autotuner)
     R *dt_elem = nullptr;                     // per-element step, or null (cfg.dt everywhere)
-    R *dt_elem_lo = nullptr;                  // its rounding
     int step = 0;
     bool have_ops = false, have_mesh = false, initialized = false;
     std::vector<char> have_mat, have_att, have_pml, have_src;
@@ -176,8 +173,6 @@ struct Batch : BatchBase {
                 (rc = dalloc(&energy, S * c.nt));
         if (!rc)
             (rc = dalloc(&matc, (size_t)nmat_sets() * c.nelem * 8)) || (rc = dalloc(&emat, (size_t)nmat_sets() * c.nelem * 2)) ||
-                (sizeof(R) == 4 && ((rc = dalloc(&mcor, (size_t)nmat_sets() * c.nelem * 4)) ||
-                                    (rc = dalloc(&matd, (size_t)nmat_sets() * c.nelem * 8)))) ||
                 (rc = dalloc(&anel, (size_t)nmat_sets() * c.nelem * nexd::NMB * 3)) ||
                 (rc = dalloc(&elist_plain, c.nelem)) || (rc = dalloc(&elist_pml, c.nelem)) || (rc = dalloc(&d_it, 1)) || (rc = dalloc(&d_done, 1)) ||
                 (rc = dalloc(&seis, S * 9 * c.nt * (c.nrec > 0 ? c.nrec : 1))) ||
@@ -272,8 +267,6 @@ struct Batch : BatchBase {
         a.nslot = nslot;
         a.scheme = cfg.timeint;
         a.dt = (R)cfg.dt;
-        a.dt_lo = (R)(cfg.dt - (double)(R)cfg.dt);
-        a.dt_elem_lo = dt_elem_lo;
         a.dt_elem = dt_elem;
         a.w13 = f32w ? (R)(1.0f / 3.0f) : (R)(1.0 / 3.0);
         a.w23 = f32w ? (R)(2.0f / 3.0f) : (R)(2.0 / 3.0);
@@ -281,7 +274,7 @@ struct Batch : BatchBase {
         a.last_flux = last_flux;
         a.last_flux1 = last_flux ? last_flux + (size_t)cfg.nshot * 27 * np : nullptr;
         a.D = D; a.DK = DK; a.LT = LT; a.fmask = fmask;
-        a.metric = metric; a.fscale = fscale; a.frame = frame; a.matc = matc; a.mcor = mcor; a.matd = matd;
+        a.metric = metric; a.fscale = fscale; a.frame = frame; a.matc = matc;
         a.nbr = nbr; a.ftype = ftype; a.anel = anel;
         for (int i = 0; i < nexd::NMB; ++i) a.wl[i] = (R)wl[i];
         a.pmlc = pmlc;
@@ -690,7 +683,7 @@ int upload_mesh(Batch<R> *b, const int *ibool, const double *const met[9], const
     if (affine) {
         b->affine_comb = ah.comb;
         if ((rc = b->put_affine_operators()) || (rc = b->upload(&b->emet, cvt<R>(ah.emet))) ||
-            (!f64 && (rc = b->upload(&b->fgeo, ah.fgeo))) || (rc = b->upload(&b->nbrt, ah.nbrt)) ||
+            (!f64 && (rc = b->upload(&b->fgeo, cvt<R>(ah.fgeo)))) || (rc = b->upload(&b->nbrt, ah.nbrt)) ||
             (f64 && ((rc = b->upload(&b->fscale, cvt<R>(m.fscale))) || (rc = b->upload(&b->frame, cvt<R>(m.frame))))))
             return rc;
     } else if ((rc = b->upload(&b->metric, cvt<R>(m.metric))) || (rc = b->upload(&b->fscale, cvt<R>(m.fscale))) ||
@@ -712,29 +705,14 @@ int upload_material(Batch<R> *b, int shot, const double *vpu, const double *vsu,
     if (rc) return rc;
     if (!vpu || !vsu || !rho || !lambdau || !muu || !mu || !lambda) return b->fail(NEXD_E_ARG, "null material");
     const int nel = b->cfg.nelem;
-    std::vector<R> mc((size_t)nel * 8, R(0)), em((size_t)nel * 2), co(sizeof(R) == 4 ? (size_t)nel * 4 : 0, R(0));
-    std::vector<double> md(sizeof(R) == 4 ? (size_t)nel * 8 : 0);
+    std::vector<R> mc((size_t)nel * 8, R(0)), em((size_t)nel * 2);
     for (int e = 0; e < nel; ++e) {
         if (!(rho[e] > 0)) return b->fail(NEXD_E_ARG, "density must be positive");
         mc[e * 8 + 0] = (R)vpu[e]; mc[e * 8 + 1] = (R)vsu[e]; mc[e * 8 + 2] = (R)rho[e];
         mc[e * 8 + 3] = (R)lambdau[e]; mc[e * 8 + 4] = (R)muu[e];
-        const double irho = 1.0 / rho[e];
-        if (sizeof(R) == 4) {
-            const double l2m = lambdau[e] + 2 * muu[e];
-            const double d[8] = {vpu[e], vsu[e], lambdau[e], muu[e], lambdau[e] * vpu[e] / l2m, irho, irho / vpu[e],
-                                 0.5 * irho / vsu[e]};
-            for (int k = 0; k < 8; ++k) md[(size_t)e * 8 + k] = d[k];
-            // as the kernel forms them: lam + 2 mu, mu, 1 / rho
-            const R l2m_r = mc[e * 8 + 3] + 2 * mc[e * 8 + 4];
-            co[e * 4 + 0] = l2m != 0 ? (R)(l2m / l2m_r - 1) : R(0);
-            co[e * 4 + 1] = muu[e] != 0 ? (R)(muu[e] / mc[e * 8 + 4] - 1) : R(0);
-            co[e * 4 + 2] = (R)(irho / (double)(R)irho - 1);
-        }
         mc[e * 8 + 5] = (R)(lambdau[e] * vpu[e] / (lambdau[e] + 2 * muu[e])); mc[e * 8 + 6] = (R)(1.0 / rho[e]);
         em[e * 2] = (R)mu[e]; em[e * 2 + 1] = (R)lambda[e];
     }
-    if (sizeof(R) == 4 && ((rc = b->put(b->mcor + (size_t)shot * nel * 4, co)) || (rc = b->put(b->matd + (size_t)shot * nel * 8, md))))
-        return rc;
     if ((rc = b->put(b->matc + (size_t)shot * nel * 8, mc)) || (rc = b->put(b->emat + (size_t)shot * nel * 2, em)))
         return rc;
     b->have_mat[shot] = 1;
@@ -866,14 +844,12 @@ int get_seis(Batch<R> *b, int shot, double *const outs[9]) {
 
 template <typename R>
 int upload_element_dt(Batch<R> *b, const double *dt_elem) {
-    std::vector<R> v(b->cfg.nelem), lo(b->cfg.nelem);
+    std::vector<R> v(b->cfg.nelem);
     for (int e = 0; e < b->cfg.nelem; ++e) {
         if (!(dt_elem[e] > 0)) return b->fail(NEXD_E_ARG, "element steps must be positive");
         v[e] = (R)dt_elem[e];
-        lo[e] = (R)(dt_elem[e] - (double)v[e]);
     }
-    int rc = b->upload(&b->dt_elem_lo, lo);
-    if (!rc) rc = b->upload(&b->dt_elem, v);
+    int rc = b->upload(&b->dt_elem, v);
     if (rc) return rc;
     b->drop_graph();
     return 0;

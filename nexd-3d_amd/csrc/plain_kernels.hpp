@@ -56,11 +56,6 @@ struct StageArgs {
     R lsa, lsb;                 // low-storage RK4: A and B of this stage
     int last_stage;             // 1 on the stage that completes a step
     R dt;
-    const double *matd;         // [nelem][8] vp vs lam mu, lam vp/(lam+2mu), 1/rho, 1/(vp rho), 1/(2 vs rho)
-    const R *mcor;              // [nelem][4] what the rounding of the material takes from the rates of the normal
-                                // stresses, shear stresses and velocities, relative (FP32 affine kernels)
-    R dt_lo;                    // its rounding, dt - (R)dt (FP32 affine kernels), and that of dt_elem
-    const R *dt_elem_lo;
     const R *dt_elem;           // [nelem] the step of each element (instances of different
                                 // step packed in one mesh) or null: dt for all
     R w13, w23;                 // RK3 final-stage weights
@@ -116,7 +111,7 @@ struct StageArgs {
     // the affine kernels' operands (affine_kernels.hpp), FP32
     const void *AK;             // [Dr|Ds|Dt|LIFT]: FP32 bfloat16 parts [step][row tile][part][64][8], FP64 [value][row tile][64]
     const R *emet;              // [nelem][12] metric (9) and padding
-    const double *fgeo;         // [nelem][4][4] normal, half the face scale (FP32)
+    const R *fgeo;              // [nelem][4][4] normal, half the face scale (FP32)
     const int *nbrt;            // [nelem][4][NPF] neighbour node, -1 free, -2 absorbing
     // compensated state (float pairs hi + lo for the 9 wavefield components
     // and the receiver-element displacement); null when not compensated
